@@ -63,7 +63,7 @@ typedef enum { W4A16_FMT_GPTQ = 0, W4A16_FMT_GPTQ_SYM = 1, W4A16_FMT_AWQ = 2 } w
  * element type, w4a16_gptq_gemm_typed.rs:65-67, and name bf16; its v0 instantiates f16).
  * A weight dequantises to RNE_bf16(f32(q - z) * f32(s)), products accumulate in fp32 and the
  * output is rounded to bf16 once. Plain group order runs the same kernels as fp16 (the
- * GEMVs, the small-batch kernel up to 64 rows, the pipelined prefill beyond; bf16 MFMA and
+ * GEMVs, the small-batch kernels up to 64 rows, the pipelined prefill beyond; bf16 MFMA and
  * v_dot2c_f32_bf16) except the block-diagonal AWQ GEMV (GPTQ at 5..8 rows takes the
  * small-batch kernel); w4a16_gemm_plan reports which; act-order runs as for fp16. Shapes
  * those kernels reject run the generic kernel. The other entry points reject
@@ -74,7 +74,8 @@ typedef enum { W4A16_FMT_GPTQ = 0, W4A16_FMT_GPTQ_SYM = 1, W4A16_FMT_AWQ = 2 } w
 typedef enum {
     W4A16_KERNEL_GEMV = 1,       /* decode: split-K GEMV, VALU dot2, no MFMA */
     W4A16_KERNEL_SKINNY = 2,     /* small batch: MFMA, weights streamed once */
-    W4A16_KERNEL_PREFILL = 3,    /* large M: dequant-to-LDS + MFMA tiles */
+    W4A16_KERNEL_PREFILL = 3,    /* more than 64 rows: MFMA tiles, weights dequantised into LDS,
+                                  * or in registers where the rows do not fill those tiles */
     W4A16_KERNEL_STRIDED = 4     /* generic strided kernel (any layout, any shape) */
 } w4a16_kernel;
 
@@ -178,7 +179,8 @@ W4A16_API int w4a16_gemm_act_order(void* stream, int fmt, const void* x, const v
  *   strip over all of K (no split-K, no scratch). With group_size a multiple of 128, 5..64 rows
  *   (4 where K <= 4096; 2..64 with perm) run a small-batch kernel, one workgroup per 1, 2 or
  *   4 strips over all of K (no split-K), which reads x (gathered by perm) as stored and puts
- *   it in the matrix cores' operand order itself.
+ *   it in the matrix cores' operand order itself. Other shapes run the kernels for more rows
+ *   on the strips, or the generic kernel.
  * w4a16_dequant_prepared: W16 as fp16 [K, N] (transposed = 0) or [N, K] (= 1), bit-exact. */
 W4A16_API size_t w4a16_prepared_bytes(int32_t K, int32_t N, int32_t group_size);
 W4A16_API int w4a16_prepare_layout(void* stream, int fmt, const void* qweight, const void* scales,

@@ -1,0 +1,103 @@
+"""GPU parity of the direct kernel (csrc/direct_body.h: weights dequantised in registers, tiles of
+16 to 112 rows) at the sizes where it can go wrong: remainders of its row and column tiles, K in
+shares that its wave groups and workgroups do not divide evenly, every group size, format, element
+type and instance. x holds whole numbers up to 2 in size and the scales are powers of two, so that
+every product and partial sum (below 2^24 units) is exact in fp32 in any order: the output must be
+the exact sum rounded once, bit for bit."""
+import numpy as np
+import pytest
+
+from helpers import pkg, to_dev
+from synth import Problem
+
+NAME = {0: "gptq", 1: "gptq_sym", 2: "awq"}
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def exact_problem(fmt, M, K, N, G, ao=False):
+    p = Problem(fmt, M=M, K=K, N=N, G=G, seed=9000 + M + K + N + G, act_order=ao)
+    g = np.random.default_rng(M * 31 + N)
+    p.x = g.integers(-2, 3, size=(M, K)).astype(np.float16)
+    p.scales = (2.0 ** -g.integers(6, 9, size=p.scales.shape)).astype(np.float16)
+    row_group = np.arange(K) // G if p.g_idx is None else p.g_idx
+    w = (p.q - p.zero_int()[row_group]) * p.scales.astype(np.float32)[row_group]
+    return p, p.x.astype(np.float32) @ w.astype(np.float32)     # exact: below 2^24 units of 2^-8
+
+
+def check(torch, y, want, dtype):
+    torch.cuda.synchronize()
+    assert torch.equal(y.cpu(), torch.from_numpy(want).to(dtype))
+
+
+CASES = [                                   # rows, N, K, group, element type
+    # AWQ, up to 64 rows: one tile of 16 R rows; one to eight splits of K
+    (2, 9, 544, 640, 64, "f16"), (2, 16, 4096, 4096, 128, "f16"), (2, 17, 1056, 4096, 256, "f16"),
+    (2, 33, 1056, 512, 32, "f16"), (2, 48, 2080, 1152, 128, "f16"), (2, 49, 6144, 1024, 64, "f16"),
+    (2, 64, 4096, 4096, 128, "bf16"), (2, 31, 512, 192, 64, "bf16"),
+    # GPTQ: wide shapes up to 64 rows, ragged widths, tiles of 64 and 112 rows by 128 and 256 columns
+    (0, 16, 20480, 256, 64, "f16"), (0, 48, 20488, 320, 32, "f16"), (0, 64, 20480, 256, 128, "bf16"),
+    (0, 65, 520, 320, 64, "f16"), (0, 113, 1096, 4096, 128, "f16"), (0, 200, 6144, 4096, 128, "f16"),
+    (1, 200, 1544, 2048, 32, "bf16"), (0, 224, 3080, 8192, 64, "f16"), (1, 700, 3072, 1024, 128, "f16"),
+    (0, 1024, 6144, 512, 128, "f16"), (1, 300, 8192, 4096, 512, "f16"), (2, 100, 1024, 4096, 128, "bf16"),
+    (2, 581, 6144, 576, 64, "f16"),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,M,N,K,G,et", CASES)
+def test_direct_bit_exact(torch_cuda, fmt, M, N, K, G, et):
+    torch = torch_cuda
+    dt = torch.float16 if et == "f16" else torch.bfloat16
+    p, want = exact_problem(fmt, M, K, N, G)
+    y = pkg().gemm(to_dev(p.x).to(dt), to_dev(p.qweight), to_dev(p.scales).to(dt),
+                   None if fmt == 1 else to_dev(p.qzeros), fmt=NAME[fmt], group_size=G)
+    check(torch, y, want, dt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,M,N,K,G", [
+    (0, 2, 528, 384, 32), (2, 20, 272, 1024, 64), (1, 70, 1040, 1024, 128), (0, 333, 1792, 4096, 64),
+    (2, 1000, 6160, 640, 128), (0, 130, 4096, 2048, 256),
+])
+def test_direct_prepared_bit_exact(torch_cuda, fmt, M, N, K, G):
+    P = pkg()
+    if fmt == 2 and N % 32:
+        N = N // 32 * 32 + 32                # the AWQ checkpoint's own width
+    p, want = exact_problem(fmt, M, K, N, G)
+    w = P.prepare_layout(to_dev(p.qweight), to_dev(p.scales), None if fmt == 1 else to_dev(p.qzeros),
+                         fmt=NAME[fmt], group_size=G, zero_offset=p.zero_offset)
+    check(torch_cuda, P.gemm_prepared(to_dev(p.x), w), want, torch_cuda.float16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,valid", [(200, 1096, 1024, True), (300, 6144, 512, True), (200, 1096, 1024, False)])
+def test_direct_behind_act_order_gate(torch_cuda, M, N, K, valid):
+    """Beyond the small-batch kernel's rows, on rows put in group order; with groups of other sizes
+    the gate leaves the output to the generic kernel."""
+    p, want = exact_problem(0, M, K, N, 128, ao=True)
+    if not valid:
+        p.g_idx = np.where(np.arange(K) == 3, (p.g_idx + 1) % (K // 128), p.g_idx).astype(np.int32)
+        w = (p.q - p.zero_int()[p.g_idx]) * p.scales.astype(np.float32)[p.g_idx]
+        want = p.x.astype(np.float32) @ w.astype(np.float32)
+    y = pkg().gemm(to_dev(p.x), to_dev(p.qweight), to_dev(p.scales), to_dev(p.qzeros), fmt="gptq",
+                   group_size=128, g_idx=to_dev(p.g_idx))
+    check(torch_cuda, y, want, torch_cuda.float16)
+
+
+def test_plan_of_widths_other_kernels_do_not_tile():
+    """Widths that no tile of the other kernels divides leave the generic kernel from 512 columns on."""
+    P = pkg()
+    for fmt, N in (("gptq", 520), ("gptq_sym", 1544), ("awq", 544)):
+        for bf16 in (False, True):
+            assert P.plan(fmt, 100, N, 640, 64, bf16=bf16) == "prefill"
+            assert P.plan(fmt, 20, N, 640, 64, bf16=bf16) == "skinny"
+    assert P.plan("gptq", 100, 504, 640, 64) == "strided"
+    assert P.plan("gptq", 100, 520, 1632, 96) == "strided"      # groups that share a stage unevenly
+    assert P.plan("gptq", 100, 520, 96, 32) == "strided"        # K that no stage divides

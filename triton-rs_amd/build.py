@@ -31,7 +31,9 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           f"-I{os.path.join(ROOT, 'include')}", f"-I{CSRC}"]
 
-SOURCES = ["api.cpp", "hiprt.cpp", "kernels_gemv.hip", "kernels_prefill.hip", "kernels_skinny.hip", "kernels_strided.hip", "kernels_moe.hip", "act_order.hip", "noalloc.hip", "prepared.hip"]
+SOURCES = ["api.cpp", "hiprt.cpp", "kernels_gemv.hip", "kernels_prefill.hip", "kernels_skinny.hip", "kernels_strided.hip", "kernels_moe.hip", "act_order.hip", "noalloc.hip", "prepared.hip",
+           "direct.hip", "direct_gptq.hip", "direct_gptq_bf16.hip", "direct_awq.hip", "direct_awq_bf16.hip",
+           "direct_prep.hip"]
 
 
 def _run(cmd):

@@ -203,6 +203,30 @@ static bool act_order_chunks_ok(int fmt, int M, int N, int K, int G) {
            ck_frag_shape(fmt, M - 64, N, K, G, true).ok;
 }
 
+// The direct kernel for a plain-order call of more than 8 rows on a checkpoint, or ok = false
+// where another kernel stays: beyond 64 rows where its modelled time is below the prefill
+// kernel's (or that has no pipelined plan); up to 64 rows for AWQ, whose small-batch kernel
+// streams 32-bit words of whole rows (M = 48: K = 4096 -> N = 4096 / 6144 / 28672 25.0 / 25.5 /
+// 42.4 -> 12.5 / 14.0 / 27.8 us), and for GPTQ from 160 tiles of 128 columns, where it needs no
+// split of K (4096 -> 28672 M = 16 / 32 / 48 24.5 / 30.5 / 46.7 -> 18.6 / 22.5 / 24.8 us; below,
+// 4096 -> 6144 M = 16 / 48 8.8 / 13.9 us against 10.3 / 15.0). Widths no tile of the others
+// divides came to the generic kernel before; narrow ones (N < 512) stay there.
+static DirectShape direct_choice(int fmt, int M, int N, int K, int G, int cus, bool bf16,
+                                 size_t max_partial_bytes = SIZE_MAX, size_t max_tiles = SPLITK_MAX_TILES) {
+    DirectShape none{};
+    if (M <= 8) return none;
+    const DirectShape ds = direct_shape(fmt, M, N, K, G, cus, bf16, max_partial_bytes, max_tiles);
+    if (!ds.ok) return none;
+    if (M > 64) {
+        const PrefillShape ps = prefill_shape(fmt, M, N, K, G, cus);
+        if (!ps.ok) return N >= 512 ? ds : none;
+        return !ps.dma || ds.us < ps.us ? ds : none;
+    }
+    const SkinnyShape sk = skinny_shape(fmt, M, N, K, G, cus);
+    if (!sk.ok || (size_t)sk.col_tiles > SPLITK_MAX_TILES) return N >= 512 ? ds : none;
+    return fmt == W4A16_FMT_AWQ || N >= 160 * 128 ? ds : none;
+}
+
 static int plan(int fmt, int M, int N, int K, int G, bool has_gidx, int cus = DEFAULT_CUS) {
     if (has_gidx) {
         const SkinnyShape sk = skinny_shape(fmt, M, N, K, G, cus, true);
@@ -216,6 +240,7 @@ static int plan(int fmt, int M, int N, int K, int G, bool has_gidx, int cus = DE
     if (M <= 64 && sk.ok && (size_t)sk.col_tiles <= SPLITK_MAX_TILES)
         return W4A16_KERNEL_SKINNY;
     if (prefill_shape(fmt, M, N, K, G, cus).ok) return W4A16_KERNEL_PREFILL;
+    if (direct_choice(fmt, M, N, K, G, cus, false).ok) return M > 64 ? W4A16_KERNEL_PREFILL : W4A16_KERNEL_SKINNY;
     return W4A16_KERNEL_STRIDED;
 }
 
@@ -234,7 +259,9 @@ static int plan_bf16(int fmt, int M, int N, int K, int G, bool has_gidx, int cus
     const SkinnyShape sk = skinny_shape(fmt, M, N, K, G, cus);
     if (M <= 64 && sk.ok && (size_t)sk.col_tiles <= SPLITK_MAX_TILES) return W4A16_KERNEL_SKINNY;
     const PrefillShape ps = prefill_shape(fmt, M, N, K, G, cus);
-    return ps.ok && ps.dma ? W4A16_KERNEL_PREFILL : W4A16_KERNEL_STRIDED;
+    if (ps.ok && ps.dma) return W4A16_KERNEL_PREFILL;
+    if (direct_choice(fmt, M, N, K, G, cus, true).ok) return M > 64 ? W4A16_KERNEL_PREFILL : W4A16_KERNEL_SKINNY;
+    return W4A16_KERNEL_STRIDED;
 }
 
 }  // namespace w4a16
@@ -316,6 +343,42 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
                       : plan(fmt, M, N, K, G, g_idx != nullptr, cus);
     if (!vec_ok) kernel = W4A16_KERNEL_STRIDED;
     if (g_idx && kernel == W4A16_KERNEL_PREFILL && !src.may_allocate) kernel = W4A16_KERNEL_STRIDED;
+    // the placement probe allocates: sources that must not allocate use what is cached
+    const bool xcd = src.may_probe ? xcd_placement(st) : xcd_placement_cached();
+    auto scratch_for = [&](size_t tiles, size_t partial_bytes, Scratch* sc) -> int {
+        if (tiles > src.max_tiles)
+            return fail(W4A16_ERR_UNSUPPORTED, "%zu split-K tiles exceed the counter area (%zu)",
+                        tiles, src.max_tiles);
+        if (partial_bytes > src.max_partial_bytes)
+            return fail(W4A16_ERR_UNSUPPORTED,
+                        "split-K partials of %zu bytes exceed the scratch limit of %zu bytes "
+                        "(M=%d N=%d K=%d)", partial_bytes, src.max_partial_bytes, M, N, K);
+        return src.get(st, partial_bytes, sc);
+    };
+    auto run_direct = [&](const DirectShape& ds, const void* xp, const void* qwp, const uint32_t* gate) -> int {
+        PrefillParams p{};
+        p.x = static_cast<const half_t*>(xp);
+        p.qweight = static_cast<const uint32_t*>(qwp);
+        p.scales = static_cast<const half_t*>(scales);
+        p.qzeros = fmt == W4A16_FMT_GPTQ_SYM ? nullptr : static_cast<const uint32_t*>(qzeros);
+        p.out = static_cast<half_t*>(out);
+        p.M = M; p.N = N; p.K = K; p.G = G; p.zero_offset = zero_offset;
+        p.gate = gate;
+        p.gate_want = 1;
+        if (ds.ksplit > 1) {
+            Scratch sc{};
+            const int r = scratch_for((size_t)ds.col_tiles * ds.row_tiles, ds.partial_bytes, &sc);
+            if (r) return r;
+            p.counters = sc.counters;
+            p.ws = sc.partials;
+        }
+        hipError_t e = launch_direct(fmt, p, ds, st, bf16);
+        return e == hipSuccess ? W4A16_OK : hip_fail(e, "direct gemm launch");
+    };
+    if (!g_idx && (kernel == W4A16_KERNEL_SKINNY || kernel == W4A16_KERNEL_PREFILL)) {
+        const DirectShape ds = direct_choice(fmt, M, N, K, G, cus, bf16, src.max_partial_bytes, src.max_tiles);
+        if (ds.ok) return run_direct(ds, x, qweight, nullptr);
+    }
     // GPTQ small batches beyond 16 rows (plain order also 9..16 with 64-column workgroups;
     // act-order also any M >= 2 with groups under 128 rows): the direct-x small-batch kernel on
     // the checkpoint as stored (one workgroup over all of K for its columns: no split-K
@@ -366,18 +429,6 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
             return e == hipSuccess ? W4A16_OK : hip_fail(e, "small-batch launch");
         }
     }
-    // the placement probe allocates: sources that must not allocate use what is cached
-    const bool xcd = src.may_probe ? xcd_placement(st) : xcd_placement_cached();
-    auto scratch_for = [&](size_t tiles, size_t partial_bytes, Scratch* sc) -> int {
-        if (tiles > src.max_tiles)
-            return fail(W4A16_ERR_UNSUPPORTED, "%zu split-K tiles exceed the counter area (%zu)",
-                        tiles, src.max_tiles);
-        if (partial_bytes > src.max_partial_bytes)
-            return fail(W4A16_ERR_UNSUPPORTED,
-                        "split-K partials of %zu bytes exceed the scratch limit of %zu bytes "
-                        "(M=%d N=%d K=%d)", partial_bytes, src.max_partial_bytes, M, N, K);
-        return src.get(st, partial_bytes, sc);
-    };
     // A fixed scratch area (w4a16_gemm_noalloc) may be too small for the split-K partials of
     // the planned GEMV or small-batch kernel (e.g. AWQ M = 8 on a 70B-class MLP: 7 MiB): such
     // a call takes the prefill kernel instead, with the largest K split whose partials fit
@@ -425,6 +476,9 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
 
     // the prefill kernel on (xp, qwp) with the call's scales and zeros; gate as PrefillParams
     auto run_prefill = [&](const void* xp, const void* qwp, const uint32_t* gate) -> int {
+        // act-order: the kernel the plain-order call takes (which came here with none)
+        if (const DirectShape ds = direct_choice(fmt, M, N, K, G, cus, bf16, src.max_partial_bytes, src.max_tiles); ds.ok)
+            return run_direct(ds, xp, qwp, gate);
         // a fixed scratch area too small for the planned split's partials: the best plan with
         // at most half the splits, down to none (no scratch at all)
         PrefillShape s = prefill_shape(fmt, M, N, K, G, cus);
@@ -729,10 +783,25 @@ W4A16_API int w4a16_gemm_prepared(void* stream, const void* x, const void* prepa
         hipError_t e = launch_prep_gemv(p, gs, st);
         return e == hipSuccess ? W4A16_OK : hip_fail(e, "prepared gemv launch");
     }
+    // more rows, or groups the small-batch kernel does not take: the direct kernel where its
+    // modelled time is below the prefill kernel's or that does not take the shape
+    const int cus = device_cus();
+    const PrefillShape pl = prefill_shape(FMT_PREP, M, N, K, G, cus);
+    const DirectShape ds = direct_shape(FMT_PREP, M, N, K, G, cus, false, SIZE_MAX, SPLITK_MAX_TILES);
+    if (ds.ok && (!(pl.ok && pl.dma) || ds.us < pl.us)) {
+        PrefillParams p{};
+        p.x = static_cast<const half_t*>(xa);
+        p.qweight = static_cast<const uint32_t*>(prepared);
+        p.out = static_cast<half_t*>(out);
+        p.M = M; p.N = N; p.K = K; p.G = G;
+        if (ds.ksplit > 1)
+            if (int rc = get_workspace(st, ds.partial_bytes, &p.counters, &p.ws)) return rc;
+        hipError_t e = launch_direct(FMT_PREP, p, ds, st);
+        return e == hipSuccess ? W4A16_OK : hip_fail(e, "prepared direct launch");
+    }
     // larger M: the pipelined prefill kernel reading the prepared strips (64-row stages: the
     // group size must be a multiple of 64; 32-bit offsets into the prepared buffer)
-    const int cus = device_cus();
-    PrefillShape ps = prefill_shape(FMT_PREP, M, N, K, G, cus);
+    PrefillShape ps = pl;
     const bool pre_ok = ps.ok && ps.dma && G % 64 == 0 && prep_total_bytes(K, N, G) < ((size_t)1 << 31);
     if (pre_ok) {
         PrefillParams p{};

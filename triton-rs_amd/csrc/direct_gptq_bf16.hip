@@ -1,0 +1,10 @@
+// Direct kernel instances: GPTQ (and GPTQ_SYM), bf16.
+#include "direct_inst.h"
+
+namespace w4a16 {
+
+hipError_t launch_direct_gptq_bf16(const PrefillParams& p, const DirectShape& s, hipStream_t st) {
+    return launch_direct_dense<FMT_GPTQ, bf16_t>(p, s, st);
+}
+
+}  // namespace w4a16

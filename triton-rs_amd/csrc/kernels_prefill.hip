@@ -846,6 +846,7 @@ PrefillShape prefill_shape(int fmt, int M, int N, int K, int G, int num_cus, int
             s.col_tiles = N / s.bn;
             s.row_tiles = (M + s.bm - 1) / s.bm;
             s.lds = prefill_dma_lds(s.bm, s.bn);
+            s.us = 4.5e-7 * best + 10.0;   // config 3: 4.7e8 units, 215-222 us
             s.ok = true;
             return s;
         }

@@ -105,6 +105,8 @@ struct PrefillParams {
     // expert-tile mode: > 0 selects the XCD-grouped workgroup order over a 1-D grid and is
     // the grid's bound on tiles (set by launch_moe_gemm_tiles)
     int xcd_tiles;
+    // direct kernel (direct_body.h): its tile counts
+    int col_tiles, row_tiles;
 };
 
 struct PrefillShape {
@@ -113,6 +115,7 @@ struct PrefillShape {
     int bm, bn, col_tiles, row_tiles;
     int ksplit;             // K splits across workgroups (1: none)
     size_t lds;
+    double us;              // pipelined kernel: the plan's modelled time
 };
 
 size_t prefill_dma_lds(int bm, int bn);
@@ -130,6 +133,19 @@ hipError_t launch_moe_gemm(int fmt, const PrefillParams& p, int block_m, int max
 bool moe_tiles_supported(int N, int K, int G, long long a_rows, int bn);
 hipError_t launch_moe_gemm_tiles(int fmt, const PrefillParams& p, int tile_bm, int bn,
                                  int max_tiles, hipStream_t st);
+
+// Direct kernel (direct_body.h): weights dequantised in registers, tiles of 16 r rows x 64 nwn
+// columns, K over kw wave groups of a workgroup and ksplit workgroups.
+struct DirectShape {
+    bool ok;
+    int r, nwn, kw, ksplit, col_tiles, row_tiles;
+    size_t partial_bytes;   // fp32 partials of the K split (0: none)
+    double us;              // modelled time
+};
+DirectShape direct_shape(int fmt, int M, int N, int K, int G, int num_cus, bool bf16,
+                         size_t max_partial_bytes, size_t max_tiles);
+// p.ws / p.counters: the split's scratch (ksplit > 1); tile counts and split are taken from s
+hipError_t launch_direct(int fmt, PrefillParams p, const DirectShape& s, hipStream_t st, bool bf16 = false);
 
 // Fused-MoE helpers (kernels_moe.hip).
 hipError_t launch_moe_route(const float* logits, int T, int E, int topk, int renormalize,

@@ -38,6 +38,14 @@ __device__ __forceinline__ void st_partial(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, SC);
 }
 
+// Four partials (16-byte aligned) as two 64-bit stores at scope SC.
+template <int SC>
+__device__ __forceinline__ void st_partial4(float* p, float4_t v) {
+    uint64_t* q = reinterpret_cast<uint64_t*>(p);
+    __hip_atomic_store(q, (uint64_t)__float_as_uint(v[0]) | ((uint64_t)__float_as_uint(v[1]) << 32), __ATOMIC_RELAXED, SC);
+    __hip_atomic_store(q + 1, (uint64_t)__float_as_uint(v[2]) | ((uint64_t)__float_as_uint(v[3]) << 32), __ATOMIC_RELAXED, SC);
+}
+
 // Four partials (16-byte aligned) as two 64-bit loads at scope SC.
 template <int SC>
 __device__ __forceinline__ float4_t ld_partial4(const float* p) {
