@@ -101,3 +101,49 @@ def test_plan_of_widths_other_kernels_do_not_tile():
     assert P.plan("gptq", 100, 504, 640, 64) == "strided"
     assert P.plan("gptq", 100, 520, 1632, 96) == "strided"      # groups that share a stage unevenly
     assert P.plan("gptq", 100, 520, 96, 32) == "strided"        # K that no stage divides
+
+
+# ------------------------------------------------------------------ by expert
+
+FEW = [0, 1, 15, 16, 17, 32, 33, 48, 49, 64]                     # tiles of up to 64 rows
+MANY = [0, 1, 17, 49, 64, 65, 80, 81, 96, 97, 112, 113, 160, 225]  # up to 112 rows, one to three each
+
+
+def expert_layer(counts, fmt, K, I, G, seed):
+    """x, logits (expert e chosen by exactly counts[e] tokens, interleaved) and stacked weights."""
+    g = np.random.default_rng(seed)
+    ids = g.permutation(np.repeat(np.arange(len(counts)), counts))
+    x = g.standard_normal((len(ids), K)).astype(np.float16)
+    logits = np.where(np.arange(len(counts)) == ids[:, None], 4.0, 0.0).astype(np.float32)
+
+    def stack(rows, cols, s):
+        ps = [Problem(fmt, M=1, K=rows, N=cols, G=G, seed=s + e) for e in range(len(counts))]
+        cat = lambda f: None if getattr(ps[0], f) is None else to_dev(np.stack([getattr(q, f) for q in ps]))
+        return cat("qweight"), cat("scales"), cat("qzeros")
+    return to_dev(x), to_dev(logits), stack(K, 2 * I, seed * 100), stack(I, K, seed * 100 + 50)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [FEW, MANY], ids=["few", "many"])
+@pytest.mark.parametrize("fmt,K,I,G", [(0, 512, 256, 64), (1, 256, 384, 64), (2, 256, 640, 128), (0, 256, 8192, 128),
+                                       (2, 256, 8192, 64)])
+def test_direct_by_expert(torch_cuda, counts, fmt, K, I, G):
+    """Experts whose rows end at the edges of the tiles. With K in one chain the layer is the
+    composition of the public pieces bit for bit; a long down projection (I = 8192) adds the sums of
+    its wave groups in another order: within the fp32 rounding of the sums, two roundings of the
+    16-bit results (h, y) and the weights' share: 2e-3 of the largest."""
+    from test_gpu_moe import _layer_by_pieces
+    P = pkg()
+    x, logits, w13, w2 = expert_layer(counts, fmt, K, I, G, 7 + fmt)
+    args = dict(topk=1, fmt=NAME[fmt], group_size=G)
+    y = P.fused_moe(x, logits, w13, w2, **args)
+    again = P.fused_moe(x, logits, w13, w2, **args)
+    want = _layer_by_pieces(P, x, logits, w13, w2, 1, NAME[fmt], G, 64)
+    assert torch_cuda.equal(y, again)
+    if I < 8192:
+        assert torch_cuda.equal(y, want)
+    prep = [y] if fmt == 1 else [y, P.fused_moe_prepared(
+        x, logits, *(P.prepare_layout_experts(*w, fmt=NAME[fmt], group_size=G) for w in (w13, w2)), topk=1)]
+    for got in prep:
+        err = (got.float() - want.float()).abs().max() / want.float().abs().max()
+        assert err.item() <= 2e-3

@@ -33,7 +33,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",
 
 SOURCES = ["api.cpp", "hiprt.cpp", "kernels_gemv.hip", "kernels_prefill.hip", "kernels_skinny.hip", "kernels_strided.hip", "kernels_moe.hip", "act_order.hip", "noalloc.hip", "prepared.hip",
            "direct.hip", "direct_gptq.hip", "direct_gptq_bf16.hip", "direct_awq.hip", "direct_awq_bf16.hip",
-           "direct_prep.hip"]
+           "direct_prep.hip", "direct_moe_gptq.hip", "direct_moe_awq.hip", "direct_moe_prep.hip"]
 
 
 def _run(cmd):

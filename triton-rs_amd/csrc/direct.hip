@@ -10,6 +10,9 @@ hipError_t launch_direct_gptq_bf16(const PrefillParams& p, const DirectShape& s,
 hipError_t launch_direct_awq(const PrefillParams& p, const DirectShape& s, hipStream_t st);
 hipError_t launch_direct_awq_bf16(const PrefillParams& p, const DirectShape& s, hipStream_t st);
 hipError_t launch_direct_prep(const PrefillParams& p, const DirectShape& s, hipStream_t st);
+hipError_t launch_direct_moe_gptq(const PrefillParams& p, const DirectShape& s, hipStream_t st);
+hipError_t launch_direct_moe_awq(const PrefillParams& p, const DirectShape& s, hipStream_t st);
+hipError_t launch_direct_moe_prep(const PrefillParams& p, const DirectShape& s, hipStream_t st);
 
 // Formats, groups and sizes the kernel reads: 32-bit byte offsets below 2^31 (offsets from 2^31 up
 // mark what reads as zero), a stage of 64 rows in whole groups or in two groups of 32
@@ -81,6 +84,40 @@ hipError_t launch_direct(int fmt, PrefillParams p, const DirectShape& s, hipStre
     if (fmt == FMT_AWQ) return bf16 ? launch_direct_awq_bf16(p, s, st) : launch_direct_awq(p, s, st);
     if (fmt == FMT_PREP && !bf16) return launch_direct_prep(p, s, st);
     return hipErrorInvalidValue;
+}
+
+// By expert: 256 columns per workgroup; where K may be summed in parts and the tiles would not give
+// every CU two workgroups, K over two groups of waves, for tiles of up to 64 rows over four, 128
+// columns wide (16 tokens, 8 experts, K = 14336 -> N = 4096: 61 us, half of it HBM's; 512 tokens:
+// 197 us against 226 us in one group)
+DirectShape direct_moe_shape(int fmt, int N, int K, int G, long long a_rows, int tile_bm, int est_tiles,
+                             int num_cus, bool split) {
+    DirectShape s{};
+    if (!direct_ok(fmt, N, K, G, a_rows) || (fmt != FMT_PREP && G % 64)) return s;
+    s.ok = true;
+    s.ksplit = 1;
+    const int ct = (N + 255) / 256;
+    const bool few = split && (long long)est_tiles * ct < 2 * num_cus;
+    s.r = few && tile_bm <= 64 ? 4 : 7;
+    s.nwn = few && tile_bm <= 64 ? 2 : 4;
+    s.kw = !few ? 1 : tile_bm <= 64 ? 4 : 2;
+    s.col_tiles = (N + 64 * s.nwn - 1) / (64 * s.nwn);
+    return s;
+}
+
+hipError_t launch_direct_moe(int fmt, PrefillParams p, const DirectShape& s, int tile_bm, int max_tiles, hipStream_t st) {
+    if (!s.ok || !p.tiles || !p.num_tiles || tile_bm > 16 * s.r || max_tiles < 1 || p.gate) return hipErrorInvalidValue;
+    p.col_tiles = s.col_tiles;
+    p.row_tiles = max_tiles;
+    p.ksplit = 1;
+    if (fmt == FMT_GPTQ_SYM) {   // as launch_direct
+        p.qzeros = nullptr;
+        p.zero_offset = 8;
+        fmt = FMT_GPTQ;
+    }
+    return fmt == FMT_GPTQ ? launch_direct_moe_gptq(p, s, st)
+           : fmt == FMT_AWQ ? launch_direct_moe_awq(p, s, st)
+           : fmt == FMT_PREP ? launch_direct_moe_prep(p, s, st) : hipErrorInvalidValue;
 }
 
 }  // namespace w4a16

@@ -40,7 +40,9 @@ constexpr int direct_bn(int nwn) { return 16 * DIR_CPL * nwn; }
 // Ring in LDS, per K group: D slots (stages), each x (16 R rows x 128 bytes) and, per wave, the
 // packed words (2 KiB) and the scales and zeros of their columns (512 bytes)
 constexpr int DIR_WST = 2048 + 512;
-constexpr int direct_depth(int r, int kw) { return r <= 2 || (r <= 4 && kw <= 2) ? 4 : 3; }
+// (four where two workgroups, or two K groups, then still fit: five row blocks and three slots left
+// an expert's K = 14336 -> N = 4096 at 205 us for 512 tokens, four slots 197)
+constexpr int direct_depth(int r, int kw) { return r <= 2 || (r <= 5 && kw <= 2) ? 4 : 3; }
 constexpr size_t direct_ring(int r, int nwn, int kw) {
     return (size_t)direct_depth(r, kw) * ((size_t)r * 16 * DIR_K * 2 + (size_t)nwn * DIR_WST);
 }
@@ -58,8 +60,25 @@ __device__ __forceinline__ void dma_lds(bufrsrc_t r, unsigned char* dst, uint32_
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, (int)voff, (int)soff, 0, 0);
 }
 
+// Workgroup b's column tile, row tile and K split. Workgroups go to the XCDs in turn (b mod 8); each
+// XCD takes an eighth of all (column tile, K split, row tile) in that order, row tiles fastest, so
+// that a column tile's weights are fetched into one L2 once, and the XCDs get equal shares whatever
+// the number of column tiles
+__device__ __forceinline__ bool direct_place(const PrefillParams& p, int rts, int& ct, int& rt, int& bz) {
+    const int total = rts * p.ksplit * p.col_tiles, share = (total + 7) >> 3;
+    const int i = blockIdx.x >> 3, idx = (blockIdx.x & 7) * share + i;
+    if (i >= share || idx >= total) return false;
+    const int u = idx / rts;
+    rt = idx - u * rts;
+    ct = u / p.ksplit;
+    bz = u - ct * p.ksplit;
+    return true;
+}
+
+// One tile: rows [m0, m0 + rows) (MOE: of the sorted pairs), 16 R at most
 template <int FMT, typename E, int R, int NWN, int KW, bool MOE>
-__global__ void __launch_bounds__(64 * NWN * KW, 2) direct_kernel(PrefillParams p) {
+__device__ __forceinline__ void direct_tile(const PrefillParams& p, unsigned char* lds, int ct, int rt, int bz,
+                                            int m0, int rows) {
     constexpr bool BF = std::is_same<E, bf16_t>::value;
     typedef typename vec8<E>::type v8_t;
     constexpr bool PREP = FMT == FMT_PREP, AWQ = FMT == FMT_AWQ;
@@ -69,42 +88,13 @@ __global__ void __launch_bounds__(64 * NWN * KW, 2) direct_kernel(PrefillParams 
     constexpr int A_ST = BM * DIR_K * 2;            // bytes of x per stage
     constexpr int DL = (2 * R + NWN - 1) / NWN;     // x loads per wave and stage (8 rows each)
     constexpr int RL = 4;                           // word loads (2), scales, zeros
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    if (p.gate && *p.gate != p.gate_want) return;   // uniform: the whole grid returns
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wn = wave % NWN, kw = wave / NWN;
     const int j = lane & 15, h = lane >> 4;
-    const int ksp = p.ksplit;
+    const int ksp = MOE ? 1 : p.ksplit;
 
-    // (column tile, row tile, K split) of this workgroup. Workgroup b runs on XCD b mod 8; the
-    // column tiles go to the XCDs in turn, all row tiles and K splits of one on the same XCD,
-    // row tiles fastest, so that its weights are fetched into one L2 once
-    int ct, rt, bz, m0, rows;
-    {
-        const int rts = MOE ? min(*p.num_tiles, p.row_tiles) : p.row_tiles;
-        if (rts <= 0) return;
-        const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
-        const int u = i / rts;
-        rt = i - u * rts;
-        const int v = u / ksp;
-        bz = u - v * ksp;
-        ct = x + 8 * v;
-        if (ct >= p.col_tiles) return;
-    }
-    if constexpr (MOE) {
-        const int32_t* td = p.tiles + 4 * rt;
-        m0 = td[0];
-        rows = td[1];
-        const int e = td[2];
-        p.qweight += (size_t)e * p.qweight_stride;
-        p.scales += (size_t)e * p.scales_stride;
-        if (p.qzeros) p.qzeros += (size_t)e * p.qzeros_stride;
-    } else {
-        m0 = rt * BM;
-        rows = min(BM, p.M - m0);
-    }
     const int n0 = ct * BN, nw0 = n0 + wn * WC;    // first column of the workgroup, the wave
     const int NW = p.N >> 3, KB = p.K / DIR_K;
     // K stages of this wave's share: [s0, s0 + ns); a stage from kend on reads zeros: its loads go
@@ -481,7 +471,7 @@ __global__ void __launch_bounds__(64 * NWN * KW, 2) direct_kernel(PrefillParams 
         }
     };
     const int lcol = PREP ? j : CPL * j;
-    if (ksp > 1) {
+    if (!MOE && ksp > 1) {
         // partials in operand order, then the last split of the tile to arrive adds all of
         // them in split order
         __shared__ int last_flag;
@@ -530,4 +520,46 @@ __global__ void __launch_bounds__(64 * NWN * KW, 2) direct_kernel(PrefillParams 
         for (int r = 0; r < R; ++r) store_rows(r, nw0 + lcol, acc[r]);
     }
 }
+
+template <int FMT, typename E, int R, int NWN, int KW>
+__global__ void __launch_bounds__(64 * NWN * KW, 2) direct_kernel(PrefillParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    if (p.gate && *p.gate != p.gate_want) return;   // uniform: the whole grid returns
+    int ct, rt, bz;
+    if (!direct_place(p, p.row_tiles, ct, rt, bz)) return;
+    direct_tile<FMT, E, R, NWN, KW, false>(p, lds, ct, rt, bz, rt * 16 * R, min(16 * R, p.M - rt * 16 * R));
+}
+
+// 8 experts of 4096 -> 28672 and 14336 -> 4096, top 2: 16 tokens 228 + 182 -> 120 + 61 us (traced;
+// the weights alone take 92 + 46 at the rate of a large copy), 512 tokens 422 + 203 -> 300 + 197 us.
+// Grouped by expert: row tile rt is entry rt of the tile list ({first sorted row, rows, expert, 0});
+// the tile's rows, known on the device only, pick the code for their number of 16-row blocks, so
+// that a tile costs what its rows need. The K groups' LDS must hold 16 RMAX rows.
+template <int FMT, int RMAX, int NWN, int KW>
+__global__ void __launch_bounds__(64 * NWN * KW, 2) direct_moe_kernel(PrefillParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int rts = min(*p.num_tiles, p.row_tiles);
+    int ct, rt, bz;
+    if (rts <= 0 || !direct_place(p, rts, ct, rt, bz)) return;
+    const int32_t* td = p.tiles + 4 * rt;
+    const int m0 = td[0], rows = td[1], e = td[2];
+    p.qweight += (size_t)e * p.qweight_stride;
+    if (FMT != FMT_PREP) {
+        p.scales += (size_t)e * p.scales_stride;
+        if (p.qzeros) p.qzeros += (size_t)e * p.qzeros_stride;
+    }
+    auto run = [&](auto r) __attribute__((always_inline)) {
+        direct_tile<FMT, half_t, decltype(r)::value, NWN, KW, true>(p, lds, ct, rt, bz, m0, rows);
+    };
+    if (rows <= 16) run(std::integral_constant<int, 1>{});
+    else if (rows <= 32) run(std::integral_constant<int, 2>{});
+    else if (rows <= 48) run(std::integral_constant<int, 3>{});
+    else if (rows <= 64) run(std::integral_constant<int, 4>{});
+    else if constexpr (RMAX > 4) {
+        if (rows <= 80) run(std::integral_constant<int, 5>{});
+        else if (rows <= 96) run(std::integral_constant<int, 6>{});
+        else run(std::integral_constant<int, 7>{});
+    }
+}
+
 }  // namespace w4a16

@@ -1,0 +1,10 @@
+// Direct kernel instances by expert: AWQ.
+#include "direct_inst.h"
+
+namespace w4a16 {
+
+hipError_t launch_direct_moe_awq(const PrefillParams& p, const DirectShape& s, hipStream_t st) {
+    return launch_direct_moe_f<FMT_AWQ>(p, s, st);
+}
+
+}  // namespace w4a16
