@@ -1210,24 +1210,31 @@ MoeTiles moe_tiles(int P, int E, int K, int I, int cus) {
     return t;
 }
 // The direct kernel for both GEMMs in place of the prefill kernel's expert tiles, in tiles of at most
-// 112 rows (64 where that holds 1.25x the mean rows per expert). It dequantises a weight once per
-// such tile, the prefill kernel once per 256 rows, and computes 16-row blocks, where the prefill
-// kernel computes its whole tile: so it stays out where tiles of 256 rows would be over 0.83 full.
+// 64 or 112 rows, whichever its time model puts lower: lower tiles where the workgroups would not
+// fill the chip. It dequantises a weight once per such tile, the prefill kernel once per 256 rows, and
+// computes 16-row blocks, where the prefill kernel computes its whole tile: so it stays out where
+// tiles of 256 rows would be over 0.83 full.
 // Measured per layer (8 experts, top 2, K = 4096, I = 14336, GPTQ; prefill tiles, direct): 4 / 16 /
 // 64 tokens 358 / 416 / 446, 149 / 192 / 200 us; 256 / 512 / 640 / 832 / 1024 tokens 477 / 556 /
 // 622 / 711 / 1037, 338 / 473 / 532 / 647 / 858 us; 864 / 960 / 1792 / 1920 (0.84 to 0.94 full)
 // 714 / 745 / 1312 / 1351, 762 / 822 / 1348 / 1484 us; 1536 / 3072 / 5000 / 8000 1181 / 2522 / 3751 /
 // 5617, 1137 / 2154 / 3563 / 5602 us.
 void moe_direct(MoeTiles& t, int fmt, int P, int T, int E, int K, int I, int G, int cus) {
-    const double mean = (double)P / E;
-    const int full = (int)((mean + std::sqrt(mean) + 255) / 256);
+    const double mean = (double)P / E, likely = mean + 0.5 * std::sqrt(mean);   // rows of an expert
+    const double full = std::ceil((mean + std::sqrt(mean)) / 256);
     if (mean > 1024 || mean > 0.83 * 256 * full) return;
-    const int bm = 1.25 * mean <= 64 ? 64 : 112;
-    const int est = E * ((int)(mean + bm - 1) / bm);
-    const DirectShape d13 = direct_moe_shape(fmt, 2 * I, K, G, T, bm, est, cus, false);
-    const DirectShape d2 = direct_moe_shape(fmt, K, I, G, P, bm, est, cus, moe_down_may_split(K, I));
-    if (!d13.ok || !d2.ok) return;
-    t.bm = bm; t.ks2 = 1; t.d13 = d13; t.d2 = d2;
+    double best = 0;
+    MoeTiles d = t;
+    for (int bm : {64, 112}) {
+        const int n = (int)std::ceil(likely / bm), rows = (int)std::ceil(likely / n), est = n * (E < P ? E : P);
+        const DirectShape d13 = direct_moe_shape(fmt, 2 * I, K, G, T, bm, est, rows, cus, false);
+        const DirectShape d2 = direct_moe_shape(fmt, K, I, G, P, bm, est, rows, cus, moe_down_may_split(K, I));
+        if (!d13.ok || !d2.ok) return;
+        if (d.d2.ok && d13.us + d2.us >= best) continue;
+        best = d13.us + d2.us;
+        d.bm = bm; d.ks2 = 1; d.d13 = d13; d.d2 = d2;
+    }
+    t = d;
 }
 }  // namespace
 

@@ -3,6 +3,8 @@
 #include "device_common.h"
 #include "launch.h"
 
+#include <cmath>
+
 namespace w4a16 {
 
 hipError_t launch_direct_gptq(const PrefillParams& p, const DirectShape& s, hipStream_t st);
@@ -91,7 +93,7 @@ hipError_t launch_direct(int fmt, PrefillParams p, const DirectShape& s, hipStre
 // columns wide (16 tokens, 8 experts, K = 14336 -> N = 4096: 61 us, half of it HBM's; 512 tokens:
 // 197 us against 226 us in one group)
 DirectShape direct_moe_shape(int fmt, int N, int K, int G, long long a_rows, int tile_bm, int est_tiles,
-                             int num_cus, bool split) {
+                             int est_rows, int num_cus, bool split) {
     DirectShape s{};
     if (!direct_ok(fmt, N, K, G, a_rows) || (fmt != FMT_PREP && G % 64)) return s;
     s.ok = true;
@@ -102,6 +104,11 @@ DirectShape direct_moe_shape(int fmt, int N, int K, int G, long long a_rows, int
     s.nwn = few && tile_bm <= 64 ? 2 : 4;
     s.kw = !few ? 1 : tile_bm <= 64 ? 4 : 2;
     s.col_tiles = (N + 64 * s.nwn - 1) / (64 * s.nwn);
+    // the dense time model's stage times (R = 5, 6 in between) for tiles of est_rows rows
+    static const double US[] = {0.42, 0.51, 0.59, 0.63, 0.72, 0.80, 0.88};
+    const double wgs = (double)est_tiles * s.col_tiles / num_cus;
+    const double load = s.kw > 1 ? std::ceil(wgs) : wgs <= 1 ? 1.0 : 0.825 * std::ceil(wgs);
+    s.us = load * ((K / 64 + s.kw - 1) / s.kw) * US[(est_rows + 15) / 16 - 1] * (s.kw > 1 ? 1.75 : 1.0);
     return s;
 }
 

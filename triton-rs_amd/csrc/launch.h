@@ -146,11 +146,12 @@ DirectShape direct_shape(int fmt, int M, int N, int K, int G, int num_cus, bool 
                          size_t max_partial_bytes, size_t max_tiles);
 // p.ws / p.counters: the split's scratch (ksplit > 1); tile counts and split are taken from s
 hipError_t launch_direct(int fmt, PrefillParams p, const DirectShape& s, hipStream_t st, bool bf16 = false);
-// By expert (p.tiles, tiles of at most tile_bm <= 112 rows, est_tiles of them expected): the instance,
-// ok = false where the kernel does not take the shape. split: K may be summed in parts (over wave
-// groups); without it the sums are those of the prefill kernel's expert tiles, bit for bit.
+// By expert (p.tiles, tiles of at most tile_bm <= 112 rows; est_tiles of est_rows rows expected): the
+// instance and its modelled time, ok = false where the kernel does not take the shape. split: K may be
+// summed in parts (over wave groups); without it the sums are those of the prefill kernel's expert
+// tiles, bit for bit.
 DirectShape direct_moe_shape(int fmt, int N, int K, int G, long long a_rows, int tile_bm, int est_tiles,
-                             int num_cus, bool split);
+                             int est_rows, int num_cus, bool split);
 hipError_t launch_direct_moe(int fmt, PrefillParams p, const DirectShape& s, int tile_bm, int max_tiles, hipStream_t st);
 
 // Fused-MoE helpers (kernels_moe.hip).
