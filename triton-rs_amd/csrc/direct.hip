@@ -46,7 +46,7 @@ DirectShape direct_shape(int fmt, int M, int N, int K, int G, int num_cus, bool 
         // up to 48 rows the tile that holds them; beyond, tiles of 64 or 112 rows
         if (M <= 48 ? c.r != (M + 15) / 16 : c.r < 4) continue;
         const int bn = 64 * c.nwn, ct = (N + bn - 1) / bn, rt = (M + 16 * c.r - 1) / (16 * c.r);
-        const double us = c.us * (bf16 ? 1.3 : 1.0) + (fmt == FMT_AWQ ? 0.06 : 0.0);
+        const double us = c.us * (bf16 ? 1.1 : 1.0) + (fmt == FMT_AWQ ? 0.06 : 0.0);
         for (int ks = 1; ks <= 8; ks *= 2) {
             // at most 8 ways, and at least four stages per wave and split
             const int ns = (K / 64 + ks * c.kw - 1) / (ks * c.kw);

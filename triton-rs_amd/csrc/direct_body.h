@@ -386,8 +386,22 @@ __device__ __forceinline__ void direct_tile(const PrefillParams& p, unsigned cha
 #pragma unroll
             for (int c = 0; c < CPL; ++c) acc[r][c] = mfma16x16x32(af[st][r], bf[st][c], acc[r][c]);
     };
+    // A step's reads and arithmetic stay inside it. Long steps are spread by hand, one MFMA to an LDS
+    // read and a share of the step's about 80 VALU instructions: the compiler's own order ends in runs
+    // of 60 VALU and 25 MFMAs, which one or two waves per SIMD do not overlap (K = 4096, GPTQ: bf16,
+    // 200 rows N = 6144 / 28672 32.8 / 72.4 -> 29.6 / 61.6 us; fp16, N = 28672 112 / 220 rows 57.4 /
+    // 60.3 -> 54.6 / 58.8 us). fp16 below five row blocks: no gain (333 rows, N = 6144 45.0, 45.7 us)
     auto order = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_barrier(0);   // a step's reads and arithmetic stay inside it
+        if constexpr (BF || R >= 5) {
+            constexpr int M = CPL * R, V = (80 + M - 1) / M;
+#pragma unroll
+            for (int i = 0; i < M; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (i < R + 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
     auto stage = [&](int s, const int u) __attribute__((always_inline)) {
         const int nx = (u + 1) % D;
