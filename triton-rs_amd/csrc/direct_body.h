@@ -390,9 +390,11 @@ __device__ __forceinline__ void direct_tile(const PrefillParams& p, unsigned cha
     // read and a share of the step's about 80 VALU instructions: the compiler's own order ends in runs
     // of 60 VALU and 25 MFMAs, which one or two waves per SIMD do not overlap (K = 4096, GPTQ: bf16,
     // 200 rows N = 6144 / 28672 32.8 / 72.4 -> 29.6 / 61.6 us; fp16, N = 28672 112 / 220 rows 57.4 /
-    // 60.3 -> 54.6 / 58.8 us). fp16 below five row blocks: no gain (333 rows, N = 6144 45.0, 45.7 us)
+    // 60.3 -> 54.6 / 58.8 us). fp16 below five row blocks: no gain (333 rows, N = 6144 45.0, 45.7 us).
+    // bf16 with one row block has too few MFMAs to spread over: left to the compiler (AWQ, 9 rows,
+    // 1792 -> 4096 / 4096 -> 6144 / 14336 -> 4096 10.0 / 15.9 / 20.4 -> 8.5 / 12.8 / 17.1 us)
     auto order = [&]() __attribute__((always_inline)) {
-        if constexpr (BF || R >= 5) {
+        if constexpr ((BF && R >= 2) || R >= 5) {
             constexpr int M = CPL * R, V = (80 + M - 1) / M;
 #pragma unroll
             for (int i = 0; i < M; ++i) {
