@@ -41,6 +41,9 @@ CASES = [                                   # rows, N, K, group, element type
     (2, 9, 544, 640, 64, "f16"), (2, 16, 4096, 4096, 128, "f16"), (2, 17, 1056, 4096, 256, "f16"),
     (2, 33, 1056, 512, 32, "f16"), (2, 48, 2080, 1152, 128, "f16"), (2, 49, 6144, 1024, 64, "f16"),
     (2, 64, 4096, 4096, 128, "bf16"), (2, 31, 512, 192, 64, "bf16"),
+    # GPTQ, 4 rows: wide shapes from K = 4096; bf16 where it stays below and from 17 rows
+    (0, 4, 20480, 4096, 128, "f16"), (1, 4, 28672, 4096, 64, "f16"),
+    (2, 9, 4096, 1792, 128, "bf16"), (0, 17, 20480, 256, 64, "bf16"),
     # GPTQ: wide shapes up to 64 rows, ragged widths, tiles of 64 and 112 rows by 128 and 256 columns
     (0, 16, 20480, 256, 64, "f16"), (0, 48, 20488, 320, 32, "f16"), (0, 64, 20480, 256, 128, "bf16"),
     (0, 65, 520, 320, 64, "f16"), (0, 113, 1096, 4096, 128, "f16"), (0, 200, 6144, 4096, 128, "f16"),

@@ -204,18 +204,21 @@ static bool act_order_chunks_ok(int fmt, int M, int N, int K, int G) {
            ck_frag_shape(fmt, M - 64, N, K, G, true).ok;
 }
 
-// The direct kernel for a plain-order call of more than 8 rows on a checkpoint, or ok = false
+// The direct kernel for a plain-order call of more than 8 rows (or 4, see below) on a checkpoint, or ok = false
 // where another kernel stays: beyond 64 rows where its modelled time is below the prefill
 // kernel's (or that has no pipelined plan); up to 64 rows for AWQ, whose small-batch kernel
 // streams 32-bit words of whole rows (M = 48: K = 4096 -> N = 4096 / 6144 / 28672 25.0 / 25.5 /
 // 42.4 -> 12.5 / 14.0 / 27.8 us), and for GPTQ from 160 tiles of 128 columns, where it needs no
 // split of K (4096 -> 28672 M = 16 / 32 / 48 24.5 / 30.5 / 46.7 -> 18.6 / 22.5 / 24.8 us; below,
-// 4096 -> 6144 M = 16 / 48 8.8 / 13.9 us against 10.3 / 15.0). Widths no tile of the others
-// divides came to the generic kernel before; narrow ones (N < 512) stay there.
+// 4096 -> 6144 M = 16 / 48 8.8 / 13.9 us against 10.3 / 15.0; in bf16 from 17 rows, 16 rows 20.7 us
+// against 23.6 on 4096 -> 20480). In fp16 also 4 rows from K = 4096, where the VALU GEMV's dot products
+// cost more (4 rows, 4096 -> 20480 / 28672, 8192 -> 28672 20.5 / 27.7 / 49.0 -> 19.5 / 21.7 / 39.7 us;
+// 2 rows 16.4 us against 21.5; 5 and 8 rows, split-K kernel, 4096 -> 20480 16.7 / 16.9 against 19.5).
+// Widths no tile of the others divides came to the generic kernel before; narrow ones (N < 512) stay there.
 static DirectShape direct_choice(int fmt, int M, int N, int K, int G, int cus, bool bf16,
                                  size_t max_partial_bytes = SIZE_MAX, size_t max_tiles = SPLITK_MAX_TILES) {
     DirectShape none{};
-    if (M <= 8) return none;
+    if (M <= 8 && (M != 4 || bf16 || fmt == W4A16_FMT_AWQ || N < 160 * 128 || K < 4096)) return none;
     const DirectShape ds = direct_shape(fmt, M, N, K, G, cus, bf16, max_partial_bytes, max_tiles);
     if (!ds.ok) return none;
     if (M > 64) {
@@ -225,6 +228,20 @@ static DirectShape direct_choice(int fmt, int M, int N, int K, int G, int cus, b
     }
     const SkinnyShape sk = skinny_shape(fmt, M, N, K, G, cus);
     if (!sk.ok || (size_t)sk.col_tiles > SPLITK_MAX_TILES) return N >= 512 ? ds : none;
+    // Up to 16 rows the direct kernel is bound by issue. AWQ: the small-batch kernel stays where its
+    // waves have at most three steps, or four and all waves run at once, one to a SIMD (M = 9 / 16: 1024 x
+    // 1024 6.24 / 6.46 against 7.17 / 7.18 us, 4096 x 4096 8.88 / 8.57 against 9.48 / 9.54; with more waves
+    // 4096 -> 6144 11.30 / 11.90 against 10.50 / 10.53, with more steps 1792 -> 4096 9.80 / 9.09 against
+    // 7.55 / 7.58). In bf16, whose weights cost half as much again, where K is split and the waves have at
+    // most ten steps (3072 x 3072 8.6 / 8.8 against 9.8, 5120 -> 12288 21.1 against 23.8 us; 14336 ->
+    // 4096, fourteen steps, 17.5 / 18.5 against 17.1, 4096 -> 28672, no split, 30.7 / 30.9 against 26.6).
+    if (M <= 16 && fmt == W4A16_FMT_AWQ) {
+        const bool resident = (long long)sk.col_tiles * sk.splits * sk.waves <= 4 * cus;
+        if (sk.steps_per_wave <= 3 || (sk.steps_per_wave <= 4 && resident)) return none;
+        if (bf16 && sk.splits > 1 && sk.steps_per_wave <= 10) return none;
+        return ds;
+    }
+    if (M <= 16 && bf16) return none;
     return fmt == W4A16_FMT_AWQ || N >= 160 * 128 ? ds : none;
 }
 
@@ -236,7 +253,8 @@ static int plan(int fmt, int M, int N, int K, int G, bool has_gidx, int cus = DE
         return act_order_prefill_ok(fmt, M, N, K, G, cus) ? W4A16_KERNEL_PREFILL : W4A16_KERNEL_STRIDED;
     }
     const GemvShape gv = gemv_shape(fmt, M, N, K, G, false);
-    if (gv.ok && (size_t)gv.col_tiles <= SPLITK_MAX_TILES) return W4A16_KERNEL_GEMV;
+    if (gv.ok && (size_t)gv.col_tiles <= SPLITK_MAX_TILES && !(M <= 8 && direct_choice(fmt, M, N, K, G, cus, false).ok))
+        return W4A16_KERNEL_GEMV;
     const SkinnyShape sk = skinny_shape(fmt, M, N, K, G, cus);
     if (M <= 64 && sk.ok && (size_t)sk.col_tiles <= SPLITK_MAX_TILES)
         return W4A16_KERNEL_SKINNY;
