@@ -36,6 +36,15 @@ SOURCES = ["api.cpp", "hiprt.cpp", "kernels_gemv.hip", "kernels_prefill.hip", "k
            "direct_prep.hip", "direct_moe_gptq.hip", "direct_moe_awq.hip", "direct_moe_prep.hip"]
 
 
+def _obj(src: str) -> str:
+    return os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+
+
+def kernel_objects() -> list[str]:
+    """The objects a program links beside its own build of the op layer (api.cpp, hiprt.cpp)."""
+    return [_obj(s) for s in SOURCES if s not in ("api.cpp", "hiprt.cpp")]
+
+
 def _run(cmd):
     r = subprocess.run(cmd, capture_output=True, text=True)
     # hipcc's host pass does not know the packed-fp32 target feature; that warning is noise
@@ -49,7 +58,7 @@ def _run(cmd):
 
 
 def _compile(src: str) -> str:
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+    obj = _obj(src)
     # .cpp sources are host code only (no device pass for a default target)
     lang = ["-x", "hip", f"--offload-arch={ARCH}"] if src.endswith(".hip") else ["--cuda-host-only"]
     _run([HIPCC, *lang, *COMMON, "-c", os.path.join(CSRC, src), "-o", obj])
@@ -58,6 +67,10 @@ def _compile(src: str) -> str:
 
 def build(verbose: bool = True) -> str:
     os.makedirs(BUILD, exist_ok=True)
+    # an object whose source is gone would still be linked by whoever takes all objects here
+    for f in os.listdir(BUILD):
+        if f.endswith(".o") and os.path.join(BUILD, f) not in map(_obj, SOURCES):
+            os.remove(os.path.join(BUILD, f))
     with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as ex:
         objs = list(ex.map(_compile, SOURCES))
         fut_hsaco = ex.submit(_run, [HIPCC, "-x", "hip", f"--offload-arch={ARCH}", *COMMON,
