@@ -19,6 +19,17 @@ def pkg():
     return __graft_entry__.load_package()
 
 
+def route(fmt, M, N, K, G, bf16=False, has_g_idx=False):
+    """The instance a call runs: ("direct", r, nwn, kw, K split), ("prefill", rows, columns, 0, K split)
+    or ("other", 0, 0, 0, 0); fmt "prep": the prepared layout beyond the kernels for few rows."""
+    import ctypes
+    P = pkg()
+    out = (ctypes.c_int32 * 5)()
+    P.lib().w4a16_internal_route((3 if fmt == "prep" else P.FORMATS[fmt]) | (P.BF16 if bf16 else 0),
+                                 M, N, K, G, int(has_g_idx), out)
+    return (("other", "direct", "prefill")[out[0]], *out[1:])
+
+
 def to_dev(a, device="cuda:0"):
     import torch
     a = np.ascontiguousarray(a)

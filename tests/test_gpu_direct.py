@@ -50,6 +50,9 @@ CASES = [                                   # rows, N, K, group, element type
     (1, 200, 1544, 2048, 32, "bf16"), (0, 224, 3080, 8192, 64, "f16"), (1, 700, 3072, 1024, 128, "f16"),
     (0, 1024, 6144, 512, 128, "f16"), (1, 300, 8192, 4096, 512, "f16"), (2, 100, 1024, 4096, 128, "bf16"),
     (2, 581, 6144, 576, 64, "f16"),
+    # many rows: rounds of workgroups on one instance
+    (0, 3072, 4096, 1792, 128, "f16"), (2, 1280, 3584, 4096, 64, "bf16"), (1, 1537, 1792, 1024, 64, "f16"),
+    (2, 3001, 1056, 1088, 32, "f16"), (0, 2100, 1096, 640, 64, "bf16"),
 ]
 
 
@@ -67,7 +70,7 @@ def test_direct_bit_exact(torch_cuda, fmt, M, N, K, G, et):
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt,M,N,K,G", [
     (0, 2, 528, 384, 32), (2, 20, 272, 1024, 64), (1, 70, 1040, 1024, 128), (0, 333, 1792, 4096, 64),
-    (2, 1000, 6160, 640, 128), (0, 130, 4096, 2048, 256),
+    (2, 1000, 6160, 640, 128), (0, 130, 4096, 2048, 256), (0, 1281, 3584, 1024, 64),
 ])
 def test_direct_prepared_bit_exact(torch_cuda, fmt, M, N, K, G):
     P = pkg()

@@ -222,9 +222,9 @@ static DirectShape direct_choice(int fmt, int M, int N, int K, int G, int cus, b
     const DirectShape ds = direct_shape(fmt, M, N, K, G, cus, bf16, max_partial_bytes, max_tiles);
     if (!ds.ok) return none;
     if (M > 64) {
-        const PrefillShape ps = prefill_shape(fmt, M, N, K, G, cus);
+        const PrefillShape ps = prefill_shape(fmt, M, N, K, G, cus, 8, bf16);
         if (!ps.ok) return N >= 512 ? ds : none;
-        return !ps.dma || ds.us < ps.us ? ds : none;
+        return direct_beats(ds, ps) ? ds : none;
     }
     const SkinnyShape sk = skinny_shape(fmt, M, N, K, G, cus);
     if (!sk.ok || (size_t)sk.col_tiles > SPLITK_MAX_TILES) return N >= 512 ? ds : none;
@@ -283,11 +283,45 @@ static int plan_bf16(int fmt, int M, int N, int K, int G, bool has_gidx, int cus
     return W4A16_KERNEL_STRIDED;
 }
 
+// The direct kernel's instance for a call whose plan is `kernel`, or ok = false: plain order beyond the
+// GEMVs; act-order on rows put in group order.
+static DirectShape planned_direct(int kernel, int fmt, int M, int N, int K, int G, bool has_gidx, int cus, bool bf16,
+                                  size_t max_partial_bytes = SIZE_MAX, size_t max_tiles = SPLITK_MAX_TILES) {
+    if (kernel == W4A16_KERNEL_PREFILL || (kernel == W4A16_KERNEL_SKINNY && !has_gidx))
+        return direct_choice(fmt, M, N, K, G, cus, bf16, max_partial_bytes, max_tiles);
+    return DirectShape{};
+}
+
+// The same on the prepared layout, for calls that neither the GEMVs nor the small-batch kernel take:
+// where its modelled time is below the prefill kernel's or that does not take the shape.
+static DirectShape prepared_direct(int M, int N, int K, int G, int cus, size_t max_partial_bytes = SIZE_MAX) {
+    const DirectShape ds = direct_shape(FMT_PREP, M, N, K, G, cus, false, max_partial_bytes, SPLITK_MAX_TILES);
+    return direct_beats(ds, prefill_shape(FMT_PREP, M, N, K, G, cus)) ? ds : DirectShape{};
+}
+
 }  // namespace w4a16
 
 using namespace w4a16;
 
 extern "C" {
+
+// Which instance a call of w4a16_gemm (fmt FMT_PREP: w4a16_gemm_prepared beyond the kernels for few
+// rows) runs, so that tests can hold a case to the instance it is for; not part of the public header.
+// out: {1, r, nwn, kw, K split} the direct kernel; {2, rows, columns, 0, K split} the pipelined prefill
+// kernel; {0} another one.
+W4A16_API void w4a16_internal_route(int fmt, int32_t M, int32_t N, int32_t K, int32_t G, int32_t has_gidx, int32_t* out) {
+    const bool bf16 = (fmt & W4A16_BF16) != 0;
+    fmt &= ~W4A16_BF16;
+    const int cus = device_cus();
+    const int kernel = fmt == FMT_PREP ? W4A16_KERNEL_PREFILL
+                       : bf16 ? plan_bf16(fmt, M, N, K, G, has_gidx != 0, cus) : plan(fmt, M, N, K, G, has_gidx != 0, cus);
+    const DirectShape ds = fmt == FMT_PREP ? prepared_direct(M, N, K, G, cus)
+                                           : planned_direct(kernel, fmt, M, N, K, G, has_gidx != 0, cus, bf16);
+    const PrefillShape ps = prefill_shape(fmt, M, N, K, G, cus);
+    const int32_t direct[5] = {1, ds.r, ds.nwn, ds.kw, ds.ksplit}, prefill[5] = {2, ps.bm, ps.bn, 0, ps.ksplit};
+    for (int i = 0; i < 5; ++i)
+        out[i] = ds.ok ? direct[i] : kernel == W4A16_KERNEL_PREFILL && ps.ok && ps.dma ? prefill[i] : 0;
+}
 
 W4A16_API const char* w4a16_last_error(void) { return g_last_error.c_str(); }
 
@@ -394,10 +428,9 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
         hipError_t e = launch_direct(fmt, p, ds, st, bf16);
         return e == hipSuccess ? W4A16_OK : hip_fail(e, "direct gemm launch");
     };
-    if (!g_idx && (kernel == W4A16_KERNEL_SKINNY || kernel == W4A16_KERNEL_PREFILL)) {
-        const DirectShape ds = direct_choice(fmt, M, N, K, G, cus, bf16, src.max_partial_bytes, src.max_tiles);
-        if (ds.ok) return run_direct(ds, x, qweight, nullptr);
-    }
+    const DirectShape ds = planned_direct(kernel, fmt, M, N, K, G, g_idx != nullptr, cus, bf16,
+                                          src.max_partial_bytes, src.max_tiles);
+    if (!g_idx && ds.ok) return run_direct(ds, x, qweight, nullptr);
     // GPTQ small batches beyond 16 rows (plain order also 9..16 with 64-column workgroups;
     // act-order also any M >= 2 with groups under 128 rows): the direct-x small-batch kernel on
     // the checkpoint as stored (one workgroup over all of K for its columns: no split-K
@@ -495,9 +528,7 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
 
     // the prefill kernel on (xp, qwp) with the call's scales and zeros; gate as PrefillParams
     auto run_prefill = [&](const void* xp, const void* qwp, const uint32_t* gate) -> int {
-        // act-order: the kernel the plain-order call takes (which came here with none)
-        if (const DirectShape ds = direct_choice(fmt, M, N, K, G, cus, bf16, src.max_partial_bytes, src.max_tiles); ds.ok)
-            return run_direct(ds, xp, qwp, gate);
+        if (ds.ok) return run_direct(ds, xp, qwp, gate);   // act-order: plain order came here with none
         // a fixed scratch area too small for the planned split's partials: the best plan with
         // at most half the splits, down to none (no scratch at all)
         PrefillShape s = prefill_shape(fmt, M, N, K, G, cus);
@@ -802,12 +833,10 @@ W4A16_API int w4a16_gemm_prepared(void* stream, const void* x, const void* prepa
         hipError_t e = launch_prep_gemv(p, gs, st);
         return e == hipSuccess ? W4A16_OK : hip_fail(e, "prepared gemv launch");
     }
-    // more rows, or groups the small-batch kernel does not take: the direct kernel where its
-    // modelled time is below the prefill kernel's or that does not take the shape
+    // more rows, or groups the small-batch kernel does not take
     const int cus = device_cus();
-    const PrefillShape pl = prefill_shape(FMT_PREP, M, N, K, G, cus);
-    const DirectShape ds = direct_shape(FMT_PREP, M, N, K, G, cus, false, SIZE_MAX, SPLITK_MAX_TILES);
-    if (ds.ok && (!(pl.ok && pl.dma) || ds.us < pl.us)) {
+    const DirectShape ds = prepared_direct(M, N, K, G, cus);
+    if (ds.ok) {
         PrefillParams p{};
         p.x = static_cast<const half_t*>(xa);
         p.qweight = static_cast<const uint32_t*>(prepared);
@@ -820,7 +849,7 @@ W4A16_API int w4a16_gemm_prepared(void* stream, const void* x, const void* prepa
     }
     // larger M: the pipelined prefill kernel reading the prepared strips (64-row stages: the
     // group size must be a multiple of 64; 32-bit offsets into the prepared buffer)
-    PrefillShape ps = pl;
+    PrefillShape ps = prefill_shape(FMT_PREP, M, N, K, G, cus);
     const bool pre_ok = ps.ok && ps.dma && G % 64 == 0 && prep_total_bytes(K, N, G) < ((size_t)1 << 31);
     if (pre_ok) {
         PrefillParams p{};

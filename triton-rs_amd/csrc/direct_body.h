@@ -1,10 +1,10 @@
-// W4A16 GEMM with the weights dequantised in registers ("direct"): from a few rows to about a
-// thousand, dense or grouped by expert. Any checkpoint format, fp16 or bf16, and the prepared
+// W4A16 GEMM with the weights dequantised in registers ("direct"): from a few rows to some thousands
+// (beyond 64 where a time model puts it ahead of the prefill kernel), dense or grouped by expert. Any checkpoint format, fp16 or bf16, and the prepared
 // layout (fp16); any N that is a multiple of 8 (AWQ 32, prepared 16), K of 64 (prepared 128),
 // groups of 32 rows or a multiple of 64.
 //
 // What it is for. The prefill kernel dequantises into LDS and shares that B tile between its
-// waves, which pays where 256-row tiles fill the chip. With 65 to a thousand rows they do not: it
+// waves, which pays where 256-row tiles fill the chip. Where they do not, mostly below a thousand rows, it
 // splits K over workgroups, and the fp32 partials (written and read back at about 4.4 TB/s) and
 // the last workgroup's sum cost more than the product. Here every wave owns 64 columns and makes
 // its own B operands (v_mfma_f32_16x16x32, 8 rows of one column per lane) from packed words, so

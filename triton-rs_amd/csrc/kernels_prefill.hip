@@ -20,6 +20,7 @@
 //
 // k order inside a chunk of 8: GPTQ words are unpacked as (k0,k4)(k1,k5)(k2,k6)(k3,k7) and
 // A is staged in that same order; AWQ keeps natural order (rows paired with v_perm_b32).
+#include <cmath>
 #include <type_traits>
 
 #include "device_common.h"
@@ -797,9 +798,28 @@ static bool dma_ok(int N, int K, int G, long long a_rows) {
            (long long)(K / G) * N * 2 < lim;
 }
 
-PrefillShape prefill_shape(int fmt, int M, int N, int K, int G, int num_cus, int max_ksplit) {
+// Modelled time of a pipelined plan, for the choice between this kernel and the one that dequantises
+// in registers: rounds of workgroups of K / 64 stages each, a stage up to 13 % faster where CUs stay
+// empty; the last round's stores; a fixed cost per round; and in a split the last workgroup's sum over
+// its tile. Fitted to graph-replay times of the plans below (30 shapes, K, N = 1024 .. 28672, M = 65 ..
+// 8192, every format, fp16 and bf16; 2800 points): nine of ten within 6 %.
+static double prefill_us(int fmt, int M, int N, int K, const PrefillShape& s, int num_cus, bool bf16) {
+    struct Tile { int bm, bn; double us, bf16, first, more; };   // us: a stage, GPTQ in fp16
+    static const Tile TILES[] = {
+        {256, 128, 1.07, 0.145, 5.2, 6.8},  {256, 192, 1.457, 0.12, 6.3, 16.6}, {256, 224, 1.512, 0.154, 7.4, 15.5},
+        {256, 256, 1.79, 0.01, 4.7, 10.5},  {128, 224, 1.28, 0.03, 6.0, 10.0},  {128, 256, 1.34, 0.03, 6.0, 10.0},
+    };
+    const Tile* t = TILES;
+    while (t->bm != s.bm || t->bn != s.bn) ++t;   // the plans' own tiles
+    const double us = t->us + (bf16 ? t->bf16 : fmt == FMT_AWQ ? 0.03 : fmt == FMT_PREP ? -0.05 : 0.0);
+    const double w = (double)s.col_tiles * s.row_tiles * s.ksplit / num_cus, n = std::ceil(w);
+    return t->first + n * (K / BK / s.ksplit) * us * (1.0 - 0.135 * (1.0 - w / n)) + t->more * (n - 1.0) +
+           0.186e-6 * 2.0 * M * N / n +
+           (s.ksplit > 1 ? 36.6e-6 * 4.0 * s.ksplit * (M < s.bm ? M : s.bm) * s.bn : 0.0);
+}
+
+PrefillShape prefill_shape(int fmt, int M, int N, int K, int G, int num_cus, int max_ksplit, bool bf16) {
     PrefillShape s{};
-    (void)fmt;
     if (M < 1 || N % 8 || K % BK || G % 8 || K % G) return s;
     if (dma_ok(N, K, G, M)) {
         // Tile (BM x BN) and K split from a cost model fitted to graph-replay times of the
@@ -846,7 +866,7 @@ PrefillShape prefill_shape(int fmt, int M, int N, int K, int G, int num_cus, int
             s.col_tiles = N / s.bn;
             s.row_tiles = (M + s.bm - 1) / s.bm;
             s.lds = prefill_dma_lds(s.bm, s.bn);
-            s.us = 4.5e-7 * best + 10.0;   // config 3: 4.7e8 units, 215-222 us
+            s.us = prefill_us(fmt, M, N, K, s, num_cus, bf16);
             s.ok = true;
             return s;
         }

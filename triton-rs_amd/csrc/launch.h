@@ -121,7 +121,9 @@ struct PrefillShape {
 size_t prefill_dma_lds(int bm, int bn);
 
 // max_ksplit caps the K split (1: never split, so no scratch is needed).
-PrefillShape prefill_shape(int fmt, int M, int N, int K, int G, int num_cus, int max_ksplit = 8);
+// bf16 enters the modelled time only
+PrefillShape prefill_shape(int fmt, int M, int N, int K, int G, int num_cus, int max_ksplit = 8,
+                           bool bf16 = false);
 // bf16: x, scales and out are bfloat16 (pipelined kernel, dense checkpoint layouts only)
 hipError_t launch_prefill(int fmt, const PrefillParams& p, const PrefillShape& s, hipStream_t st,
                           bool bf16 = false);
@@ -144,6 +146,10 @@ struct DirectShape {
 };
 DirectShape direct_shape(int fmt, int M, int N, int K, int G, int num_cus, bool bf16,
                          size_t max_partial_bytes, size_t max_tiles);
+// Beyond 64 rows: whether it takes the prefill kernel's place. 3 % in doubt stay with that one.
+inline bool direct_beats(const DirectShape& ds, const PrefillShape& ps) {
+    return ds.ok && (!(ps.ok && ps.dma) || 1.03 * ds.us < ps.us);
+}
 // p.ws / p.counters: the split's scratch (ksplit > 1); tile counts and split are taken from s
 hipError_t launch_direct(int fmt, PrefillParams p, const DirectShape& s, hipStream_t st, bool bf16 = false);
 // By expert (p.tiles, tiles of at most tile_bm <= 112 rows; est_tiles of est_rows rows expected): the
