@@ -7,7 +7,7 @@ the exact sum rounded once, bit for bit."""
 import numpy as np
 import pytest
 
-from helpers import pkg, to_dev
+from helpers import pkg, route, to_dev
 from synth import Problem
 
 NAME = {0: "gptq", 1: "gptq_sym", 2: "awq"}
@@ -153,3 +153,51 @@ def test_direct_by_expert(torch_cuda, counts, fmt, K, I, G):
     for got in prep:
         err = (got.float() - want.float()).abs().max() / want.float().abs().max()
         assert err.item() <= 2e-3
+
+
+# ------------------------------------------------------------------ under capture
+
+def fresh_stream(torch):
+    """A stream the library has not seen (torch's own streams come from a pool and are reused)."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    h = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(h)) == 0
+    return torch.cuda.ExternalStream(h.value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,M,N,K,warm", [
+    (0, 48, 1032, 4096, 0), (2, 17, 1056, 4096, 0), (0, 113, 1096, 4096, 0), ("prep", 80, 1040, 2048, 0),
+    (0, 333, 4104, 14336, 9), (2, 200, 3104, 14336, 9)])
+def test_direct_captured_without_its_workspace(torch_cuda, fmt, M, N, K, warm):
+    """A call that splits K, captured on a stream with no workspace or one too small for the split (that
+    of a call of `warm` rows), runs with fewer splits instead of asking for one."""
+    torch, P = torch_cuda, pkg()
+    prep = fmt == "prep"
+    f = 0 if prep else fmt
+    assert route("prep" if prep else NAME[f], M, N, K, 128)[0] == "direct"
+    assert route("prep" if prep else NAME[f], M, N, K, 128)[4] > 1
+    p, want = exact_problem(f, M, K, N, 128)
+    x, qw, sc, qz = (to_dev(v) for v in (p.x, p.qweight, p.scales, p.qzeros))
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda:0")
+    w = P.prepare_layout(qw, sc, qz, fmt="gptq", group_size=128) if prep else None
+    s = fresh_stream(torch)
+
+    def call(xs, o):
+        if prep:
+            P.gemm_prepared(xs, w, out=o)
+        else:
+            P.gemm(xs, qw, sc, qz, fmt=NAME[f], group_size=128, out=o)
+    if warm:
+        with torch.cuda.stream(s):
+            call(x[:warm], out[:warm])
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(x, out)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        check(torch, out, want, torch.float16)

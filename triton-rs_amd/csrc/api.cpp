@@ -100,6 +100,21 @@ static int get_workspace(hipStream_t st, size_t need, uint32_t** counters, float
     return W4A16_OK;
 }
 
+// Limit on the split-K partials of a call that would use `need` bytes of them where an unsplit plan
+// exists: none, but while the stream is captured with a smaller workspace, what that holds (a plan that
+// fits then takes the place of one whose workspace cannot be allocated).
+static size_t partials_limit(hipStream_t st, size_t need) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return SIZE_MAX; }
+    size_t have = 0;
+    {
+        std::lock_guard<std::mutex> lk(g_ws_mu);
+        auto it = g_ws.find({dev, st});
+        if (it != g_ws.end() && it->second.bytes > COUNTER_BYTES) have = it->second.bytes - COUNTER_BYTES;
+    }
+    return have >= need || !stream_capturing(st) ? SIZE_MAX : have;
+}
+
 // Per-(device, stream) buffer for activations gathered into act-order group order.
 static std::map<std::pair<int, hipStream_t>, Workspace> g_gather;
 // act-order beyond 64 rows on w4a16_gemm: perm, the gate word and the repacked rows
@@ -428,8 +443,12 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
         hipError_t e = launch_direct(fmt, p, ds, st, bf16);
         return e == hipSuccess ? W4A16_OK : hip_fail(e, "direct gemm launch");
     };
-    const DirectShape ds = planned_direct(kernel, fmt, M, N, K, G, g_idx != nullptr, cus, bf16,
-                                          src.max_partial_bytes, src.max_tiles);
+    DirectShape ds = planned_direct(kernel, fmt, M, N, K, G, g_idx != nullptr, cus, bf16,
+                                    src.max_partial_bytes, src.max_tiles);
+    if (ds.ksplit > 1 && src.may_allocate) {
+        const size_t lim = partials_limit(st, ds.partial_bytes);
+        if (lim != SIZE_MAX) ds = planned_direct(kernel, fmt, M, N, K, G, g_idx != nullptr, cus, bf16, lim, src.max_tiles);
+    }
     if (!g_idx && ds.ok) return run_direct(ds, x, qweight, nullptr);
     // GPTQ small batches beyond 16 rows (plain order also 9..16 with 64-column workgroups;
     // act-order also any M >= 2 with groups under 128 rows): the direct-x small-batch kernel on
@@ -835,7 +854,11 @@ W4A16_API int w4a16_gemm_prepared(void* stream, const void* x, const void* prepa
     }
     // more rows, or groups the small-batch kernel does not take
     const int cus = device_cus();
-    const DirectShape ds = prepared_direct(M, N, K, G, cus);
+    DirectShape ds = prepared_direct(M, N, K, G, cus);
+    if (ds.ksplit > 1) {
+        const size_t lim = partials_limit(st, ds.partial_bytes);
+        if (lim != SIZE_MAX) ds = prepared_direct(M, N, K, G, cus, lim);
+    }
     if (ds.ok) {
         PrefillParams p{};
         p.x = static_cast<const half_t*>(xa);
