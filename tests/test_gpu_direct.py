@@ -201,3 +201,44 @@ def test_direct_captured_without_its_workspace(torch_cuda, fmt, M, N, K, warm):
         torch.cuda.synchronize()
         g.replay()
         check(torch, out, want, torch.float16)
+
+
+BESIDE_A_CAPTURE = """
+import sys
+sys.path[:0] = [{root!r}, {tests!r}]
+import torch
+from helpers import pkg, to_dev
+from test_gpu_direct import exact_problem
+P = pkg()
+p, want = exact_problem({fmt}, {M}, {K}, {N}, 128)
+args = [to_dev(v) for v in (p.x, p.qweight, p.scales, p.qzeros)]
+out = torch.zeros(({M}, {N}), dtype=torch.float16, device="cuda")
+y = torch.zeros(16, device="cuda")
+a, b = torch.cuda.Stream(), torch.cuda.Stream()
+torch.cuda.synchronize()
+g = torch.cuda.CUDAGraph()
+with torch.cuda.graph(g, stream=a):
+    y.add_(1)
+    with torch.cuda.stream(b):
+        P.gemm(*args, fmt={name!r}, out=out)
+g.replay()
+torch.cuda.synchronize()
+assert torch.equal(out.cpu(), torch.from_numpy(want).to(torch.float16)) and y.eq(1).all()
+print("both right")
+"""
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,M,K,N", [(0, 48, 512, 512), (2, 33, 512, 1056)], ids=["small-batch", "direct"])
+def test_first_call_beside_a_capture(torch_cuda, fmt, M, K, N):
+    """The first call of a process, on the kernels that use neither scratch nor the workgroups'
+    placement, allocates nothing: a capture on another stream, which an allocation would
+    invalidate, goes on."""
+    import os
+    import subprocess
+    import sys
+    from helpers import ROOT
+    assert fmt == 0 or route(NAME[fmt], M, N, K, 128) == ("direct", 3, 2, 2, 1)
+    src = BESIDE_A_CAPTURE.format(root=ROOT, tests=os.path.join(ROOT, "tests"), fmt=fmt, M=M, K=K, N=N, name=NAME[fmt])
+    r = subprocess.run([sys.executable, "-c", src], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "both right" in r.stdout, r.stderr[-1500:]

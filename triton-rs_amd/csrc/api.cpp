@@ -411,8 +411,6 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
                       : plan(fmt, M, N, K, G, g_idx != nullptr, cus);
     if (!vec_ok) kernel = W4A16_KERNEL_STRIDED;
     if (g_idx && kernel == W4A16_KERNEL_PREFILL && !src.may_allocate) kernel = W4A16_KERNEL_STRIDED;
-    // the placement probe allocates: sources that must not allocate use what is cached
-    const bool xcd = src.may_probe ? xcd_placement(st) : xcd_placement_cached();
     auto scratch_for = [&](size_t tiles, size_t partial_bytes, Scratch* sc) -> int {
         if (tiles > src.max_tiles)
             return fail(W4A16_ERR_UNSUPPORTED, "%zu split-K tiles exceed the counter area (%zu)",
@@ -500,6 +498,9 @@ int gemm_impl(void* stream, int fmt, const void* x, const void* qweight, const v
             return e == hipSuccess ? W4A16_OK : hip_fail(e, "small-batch launch");
         }
     }
+    // The placement probe allocates: sources that must not allocate use what is cached, and the kernels
+    // above, which do not need it, run without (an allocation invalidates captures on other streams).
+    const bool xcd = src.may_probe ? xcd_placement(st) : xcd_placement_cached();
     // A fixed scratch area (w4a16_gemm_noalloc) may be too small for the split-K partials of
     // the planned GEMV or small-batch kernel (e.g. AWQ M = 8 on a 70B-class MLP: 7 MiB): such
     // a call takes the prefill kernel instead, with the largest K split whose partials fit
