@@ -162,14 +162,20 @@ def test_typed_code_object_names_and_metadata():
         assert k["params"] == 21
 
 
-def _disassemble_tu(obj, tmp_path):
-    """gfx950 disassembly of one of our own build's translation units."""
+def _device_object(obj, tmp_path):
+    """The gfx950 code object of one of our own build's translation units."""
     fb, dev = tmp_path / "fb.bin", tmp_path / "dev.o"
     subprocess.run(["objcopy", "-O", "binary", "--only-section=.hip_fatbin", obj, str(fb)],
                    check=True)
     subprocess.run(["/opt/rocm/llvm/bin/clang-offload-bundler", "--unbundle", "--type=o",
                     "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={fb}",
                     f"--output={dev}"], check=True)
+    return dev
+
+
+def _disassemble_tu(obj, tmp_path):
+    """gfx950 disassembly of one of our own build's translation units."""
+    dev = _device_object(obj, tmp_path)
     dis = subprocess.run(["/opt/rocm/llvm/bin/llvm-objdump", "-d", str(dev)],
                          capture_output=True, text=True, check=True).stdout
     funcs = {}
@@ -470,3 +476,20 @@ def test_gemm_prepared_python_refuses_perm_with_g_idx():
     i = torch.empty(4096, dtype=torch.int32)
     with pytest.raises(P.InvalidArgument, match="not both"):
         P.gemm_prepared(x, w, perm=i, g_idx=i)
+
+
+def test_direct_kernels_lds_and_registers(tmp_path):
+    """The expert instances of the direct kernel fill the 160 KiB of LDS with their rings: no static
+    LDS beside them (the dense ones hold one flag). None spills to scratch."""
+    bdir = os.path.join(ROOT, "triton-rs_amd", "_build")
+    names = ("gptq", "gptq_bf16", "awq", "awq_bf16", "prep", "moe_gptq", "moe_awq", "moe_prep")
+    objs = [os.path.join(bdir, f"direct_{n}.o") for n in names]
+    if not all(os.path.exists(o) for o in objs):
+        pytest.skip("build objects not present (run build first)")
+    for name, o in zip(names, objs):
+        notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", str(_device_object(o, tmp_path))],
+                               capture_output=True, text=True, check=True).stdout
+        lds = [int(v) for v in re.findall(r"\.group_segment_fixed_size: (\d+)", notes)]
+        scratch = [int(v) for v in re.findall(r"\.private_segment_fixed_size: (\d+)", notes)]
+        assert len(lds) == len(scratch) == (3 if "moe" in name else 7), name
+        assert max(lds) <= (0 if "moe" in name else 64) and max(scratch) == 0, (name, lds, scratch)

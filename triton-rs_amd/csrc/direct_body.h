@@ -487,7 +487,7 @@ __device__ __forceinline__ void direct_tile(const PrefillParams& p, unsigned cha
         }
     };
     const int lcol = PREP ? j : CPL * j;
-    if (!MOE && ksp > 1) {
+    if constexpr (!MOE) if (ksp > 1) {   // not by expert: no room for the flag beside 160 KiB of rings
         // partials in operand order, then the last split of the tile to arrive adds all of
         // them in split order
         __shared__ int last_flag;
