@@ -1,7 +1,7 @@
 """GPU parity of the direct kernel (csrc/direct_body.h: weights dequantised in registers, tiles of
 16 to 112 rows) at the sizes where it can go wrong: remainders of its row and column tiles, K in
 shares that its wave groups and workgroups do not divide evenly, every group size, format, element
-type and instance. x holds whole numbers up to 2 in size and the scales are powers of two, so that
+type and instance (each case names its own, which a test without GPU holds it to). x holds whole numbers up to 2 in size and the scales are powers of two, so that
 every product and partial sum (below 2^24 units) is exact in fp32 in any order: the output must be
 the exact sum rounded once, bit for bit."""
 import numpy as np
@@ -36,29 +36,75 @@ def check(torch, y, want, dtype):
     assert torch.equal(y.cpu(), torch.from_numpy(want).to(dtype))
 
 
-CASES = [                                   # rows, N, K, group, element type
+CASES = [                                   # rows, N, K, group, element type, instance
     # AWQ, up to 64 rows: one tile of 16 R rows; one to eight splits of K
-    (2, 9, 544, 640, 64, "f16"), (2, 16, 4096, 4096, 128, "f16"), (2, 17, 1056, 4096, 256, "f16"),
-    (2, 33, 1056, 512, 32, "f16"), (2, 48, 2080, 1152, 128, "f16"), (2, 49, 6144, 1024, 64, "f16"),
-    (2, 64, 4096, 4096, 128, "bf16"), (2, 31, 512, 192, 64, "bf16"),
+    (2, 9, 544, 640, 64, "f16", "1x2x2/1"), (2, 16, 4096, 4096, 128, "f16", "other"),
+    (2, 17, 1056, 4096, 256, "f16", "2x2x2/8"),
+    (2, 33, 1056, 512, 32, "f16", "3x2x2/1"), (2, 48, 2080, 1152, 128, "f16", "3x2x2/2"),
+    (2, 49, 6144, 1024, 64, "f16", "4x2x2/1"),
+    (2, 64, 4096, 4096, 128, "bf16", "4x2x2/4"), (2, 31, 512, 192, 64, "bf16", "2x2x2/1"),
     # GPTQ, 4 rows: wide shapes from K = 4096; bf16 where it stays below and from 17 rows
-    (0, 4, 20480, 4096, 128, "f16"), (1, 4, 28672, 4096, 64, "f16"),
-    (2, 9, 4096, 1792, 128, "bf16"), (0, 17, 20480, 256, 64, "bf16"),
+    (0, 4, 20480, 4096, 128, "f16", "1x2x2/1"), (1, 4, 28672, 4096, 64, "f16", "1x2x2/1"),
+    (2, 9, 4096, 1792, 128, "bf16", "other"), (0, 17, 20480, 256, 64, "bf16", "2x2x2/1"),
     # GPTQ: wide shapes up to 64 rows, ragged widths, tiles of 64 and 112 rows by 128 and 256 columns
-    (0, 16, 20480, 256, 64, "f16"), (0, 48, 20488, 320, 32, "f16"), (0, 64, 20480, 256, 128, "bf16"),
-    (0, 65, 520, 320, 64, "f16"), (0, 113, 1096, 4096, 128, "f16"), (0, 200, 6144, 4096, 128, "f16"),
-    (1, 200, 1544, 2048, 32, "bf16"), (0, 224, 3080, 8192, 64, "f16"), (1, 700, 3072, 1024, 128, "f16"),
-    (0, 1024, 6144, 512, 128, "f16"), (1, 300, 8192, 4096, 512, "f16"), (2, 100, 1024, 4096, 128, "bf16"),
-    (2, 581, 6144, 576, 64, "f16"),
+    (0, 16, 20480, 256, 64, "f16", "1x2x2/1"), (0, 48, 20488, 320, 32, "f16", "3x2x2/1"),
+    (0, 64, 20480, 256, 128, "bf16", "4x2x2/1"),
+    (0, 65, 520, 320, 64, "f16", "4x2x2/1"), (0, 113, 1096, 4096, 128, "f16", "4x2x2/8"),
+    (0, 200, 6144, 4096, 128, "f16", "4x2x4/1"),
+    (1, 200, 1544, 2048, 32, "bf16", "4x2x2/4"), (0, 224, 3080, 8192, 64, "f16", "4x2x4/2"),
+    (1, 700, 3072, 1024, 128, "f16", "7x2x2/1"),
+    (0, 1024, 6144, 512, 128, "f16", "7x4x1/1"), (1, 300, 8192, 4096, 512, "f16", "7x2x2/1"),
+    (2, 100, 1024, 4096, 128, "bf16", "4x2x2/8"),
+    (2, 581, 6144, 576, 64, "f16", "7x4x1/1"),
     # many rows: rounds of workgroups on one instance
-    (0, 3072, 4096, 1792, 128, "f16"), (2, 1280, 3584, 4096, 64, "bf16"), (1, 1537, 1792, 1024, 64, "f16"),
-    (2, 3001, 1056, 1088, 32, "f16"), (0, 2100, 1096, 640, 64, "bf16"),
+    (0, 3072, 4096, 1792, 128, "f16", "7x4x1/1"), (2, 1280, 3584, 4096, 64, "bf16", "7x4x1/1"),
+    (1, 1537, 1792, 1024, 64, "f16", "7x2x2/1"),
+    (2, 3001, 1056, 1088, 32, "f16", "7x2x2/1"), (0, 2100, 1096, 640, 64, "bf16", "7x2x2/1"),
+]
+
+# every instance in both formats and element types, without and with K split over workgroups
+INSTANCES = [
+    (0, 9, 544, 192, 64, "f16", "1x2x2/1"), (0, 9, 544, 1984, 64, "f16", "1x2x2/4"),
+    (0, 17, 544, 192, 64, "f16", "2x2x2/1"), (0, 17, 544, 1984, 64, "f16", "2x2x2/4"),
+    (0, 33, 544, 192, 64, "f16", "3x2x2/1"), (0, 33, 544, 1088, 64, "f16", "3x2x2/2"),
+    (0, 49, 544, 192, 64, "f16", "4x2x2/1"), (0, 49, 544, 1088, 64, "f16", "4x2x2/2"),
+    (0, 65, 6176, 1984, 64, "f16", "4x2x4/1"), (0, 400, 544, 5888, 64, "f16", "4x2x4/4"),
+    (0, 200, 8224, 320, 64, "f16", "7x2x2/1"), (0, 200, 2080, 6848, 64, "f16", "7x2x2/4"),
+    (0, 200, 8224, 192, 64, "f16", "7x4x1/1"), (0, 447, 3616, 11968, 64, "f16", "7x4x1/4"),
+    (0, 9, 544, 192, 64, "bf16", "1x2x2/1"), (0, 9, 544, 1088, 64, "bf16", "1x2x2/2"),
+    (0, 17, 544, 192, 64, "bf16", "2x2x2/1"), (0, 17, 544, 1088, 64, "bf16", "2x2x2/2"),
+    (0, 33, 544, 192, 64, "bf16", "3x2x2/1"), (0, 33, 544, 1088, 64, "bf16", "3x2x2/2"),
+    (0, 49, 544, 192, 64, "bf16", "4x2x2/1"), (0, 49, 544, 1088, 64, "bf16", "4x2x2/2"),
+    (0, 65, 8224, 1984, 64, "bf16", "4x2x4/1"), (0, 400, 544, 6848, 64, "bf16", "4x2x4/4"),
+    (0, 200, 8224, 320, 64, "bf16", "7x2x2/1"), (0, 200, 2080, 3968, 64, "bf16", "7x2x2/4"),
+    (0, 200, 8224, 192, 64, "bf16", "7x4x1/1"), (0, 200, 8224, 12288, 64, "bf16", "7x4x1/2"),
+    (2, 9, 544, 192, 64, "f16", "1x2x2/1"), (2, 9, 544, 1984, 64, "f16", "1x2x2/4"),
+    (2, 17, 544, 192, 64, "f16", "2x2x2/1"), (2, 17, 544, 1088, 64, "f16", "2x2x2/2"),
+    (2, 33, 544, 192, 64, "f16", "3x2x2/1"), (2, 33, 544, 1088, 64, "f16", "3x2x2/2"),
+    (2, 49, 544, 192, 64, "f16", "4x2x2/1"), (2, 49, 544, 1088, 64, "f16", "4x2x2/2"),
+    (2, 1300, 544, 1984, 64, "f16", "4x2x4/1"), (2, 400, 544, 6848, 64, "f16", "4x2x4/4"),
+    (2, 200, 8224, 320, 64, "f16", "7x2x2/1"), (2, 65, 4128, 4608, 64, "f16", "7x2x2/4"),
+    (2, 200, 8224, 192, 64, "f16", "7x4x1/1"), (2, 447, 3616, 12288, 64, "f16", "7x4x1/4"),
+    (2, 9, 544, 192, 64, "bf16", "1x2x2/1"), (2, 9, 544, 1088, 64, "bf16", "1x2x2/2"),
+    (2, 17, 544, 192, 64, "bf16", "2x2x2/1"), (2, 17, 544, 1088, 64, "bf16", "2x2x2/2"),
+    (2, 33, 544, 192, 64, "bf16", "3x2x2/1"), (2, 33, 544, 1088, 64, "bf16", "3x2x2/2"),
+    (2, 49, 544, 192, 64, "bf16", "4x2x2/1"), (2, 49, 544, 1088, 64, "bf16", "4x2x2/2"),
+    (2, 900, 1056, 1984, 64, "bf16", "4x2x4/1"), (2, 400, 544, 6848, 64, "bf16", "4x2x4/4"),
+    (2, 200, 8224, 320, 64, "bf16", "7x2x2/1"), (2, 200, 2080, 3648, 64, "bf16", "7x2x2/4"),
+    (2, 200, 8224, 192, 64, "bf16", "7x4x1/1"), (2, 223, 8224, 11968, 64, "bf16", "7x4x1/2"),
 ]
 
 
+@pytest.mark.parametrize("fmt,M,N,K,G,et,instance", CASES + INSTANCES)
+def test_cases_take_their_instance(fmt, M, N, K, G, et, instance):
+    """R x waves along N x wave groups along K / K split ("other": not the direct kernel). No GPU."""
+    kind, *shape = route(NAME[fmt], M, N, K, G, et == "bf16")
+    assert instance == ("{}x{}x{}/{}".format(*shape) if kind == "direct" else "other")
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("fmt,M,N,K,G,et", CASES)
-def test_direct_bit_exact(torch_cuda, fmt, M, N, K, G, et):
+@pytest.mark.parametrize("fmt,M,N,K,G,et,instance", CASES + INSTANCES)
+def test_direct_bit_exact(torch_cuda, fmt, M, N, K, G, et, instance):
     torch = torch_cuda
     dt = torch.float16 if et == "f16" else torch.bfloat16
     p, want = exact_problem(fmt, M, K, N, G)
@@ -67,12 +113,28 @@ def test_direct_bit_exact(torch_cuda, fmt, M, N, K, G, et):
     check(torch, y, want, dt)
 
 
+PREPARED = [    # checkpoint format, rows, N, K, group; instance (groups under 128 and 9 rows or more, or 65)
+    (0, 2, 528, 384, 32, "other"), (2, 20, 272, 1024, 64, "2x2x2/2"), (1, 70, 1040, 1024, 128, "4x2x2/2"),
+    (0, 333, 1792, 4096, 64, "4x2x4/2"), (2, 1000, 6160, 640, 128, "7x4x1/1"), (0, 130, 4096, 2048, 256, "4x2x2/2"),
+    (0, 1281, 3584, 1024, 64, "7x4x1/1"),
+    # every instance, without and with K split over workgroups
+    (0, 9, 528, 128, 64, "1x2x2/1"), (0, 9, 528, 1920, 64, "1x2x2/4"), (0, 17, 528, 128, 64, "2x2x2/1"),
+    (0, 33, 528, 128, 64, "3x2x2/1"), (0, 33, 528, 1152, 32, "3x2x2/2"), (0, 49, 528, 128, 64, "4x2x2/1"),
+    (0, 65, 4112, 4096, 64, "4x2x4/2"), (0, 200, 8208, 256, 64, "7x2x2/1"), (0, 65, 4112, 6272, 64, "7x2x2/4"),
+    (0, 200, 8208, 12288, 64, "7x4x1/2"),
+]
+
+
+@pytest.mark.parametrize("fmt,M,N,K,G,instance", PREPARED)
+def test_prepared_cases_take_their_instance(fmt, M, N, K, G, instance):
+    if instance != "other":              # that one: the GEMV for few rows
+        kind, *shape = route("prep", M, (N + 31) // 32 * 32 if fmt == 2 else N, K, G)
+        assert kind == "direct" and instance == "{}x{}x{}/{}".format(*shape)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("fmt,M,N,K,G", [
-    (0, 2, 528, 384, 32), (2, 20, 272, 1024, 64), (1, 70, 1040, 1024, 128), (0, 333, 1792, 4096, 64),
-    (2, 1000, 6160, 640, 128), (0, 130, 4096, 2048, 256), (0, 1281, 3584, 1024, 64),
-])
-def test_direct_prepared_bit_exact(torch_cuda, fmt, M, N, K, G):
+@pytest.mark.parametrize("fmt,M,N,K,G,instance", PREPARED)
+def test_direct_prepared_bit_exact(torch_cuda, fmt, M, N, K, G, instance):
     P = pkg()
     if fmt == 2 and N % 32:
         N = N // 32 * 32 + 32                # the AWQ checkpoint's own width
@@ -82,19 +144,27 @@ def test_direct_prepared_bit_exact(torch_cuda, fmt, M, N, K, G):
     check(torch_cuda, P.gemm_prepared(to_dev(p.x), w), want, torch_cuda.float16)
 
 
+GATED = [(200, 1096, 1024, True), (300, 6144, 512, True), (200, 1096, 1024, False),
+         (300, 6144, 512, False), (150, 1024, 4096, True), (150, 1024, 4096, False)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,valid", [(200, 1096, 1024, True), (300, 6144, 512, True), (200, 1096, 1024, False)])
+@pytest.mark.parametrize("M,N,K,valid", GATED)
 def test_direct_behind_act_order_gate(torch_cuda, M, N, K, valid):
-    """Beyond the small-batch kernel's rows, on rows put in group order; with groups of other sizes
-    the gate leaves the output to the generic kernel."""
+    """Beyond the small-batch kernel's rows, on rows put in group order (K whole, K split over
+    workgroups); with groups of other sizes the gate leaves the output to the generic kernel. Widths
+    without a prefill plan (1096) go to that one at once."""
+    kind, _, _, _, split = route("gptq", M, N, K, 128, has_g_idx=True)
+    assert kind == ("other" if N == 1096 else "direct") and (split > 1) == (K == 4096)
     p, want = exact_problem(0, M, K, N, 128, ao=True)
     if not valid:
         p.g_idx = np.where(np.arange(K) == 3, (p.g_idx + 1) % (K // 128), p.g_idx).astype(np.int32)
         w = (p.q - p.zero_int()[p.g_idx]) * p.scales.astype(np.float32)[p.g_idx]
         want = p.x.astype(np.float32) @ w.astype(np.float32)
-    y = pkg().gemm(to_dev(p.x), to_dev(p.qweight), to_dev(p.scales), to_dev(p.qzeros), fmt="gptq",
-                   group_size=128, g_idx=to_dev(p.g_idx))
-    check(torch_cuda, y, want, torch_cuda.float16)
+    args = [to_dev(v) for v in (p.x, p.qweight, p.scales, p.qzeros)]
+    for _ in range(2):                       # the split's counters are left at zero either way
+        y = pkg().gemm(*args, fmt="gptq", group_size=128, g_idx=to_dev(p.g_idx))
+        check(torch_cuda, y, want, torch_cuda.float16)
 
 
 def test_plan_of_widths_other_kernels_do_not_tile():
