@@ -30,6 +30,16 @@ def route(fmt, M, N, K, G, bf16=False, has_g_idx=False):
     return (("other", "direct", "prefill")[out[0]], *out[1:])
 
 
+def moe_route(fmt, T, K, I, E, topk, G):
+    """What the expert GEMMs of a fused layer run: ("direct", tile rows, (r, nwn, kw) of gate/up, of down)
+    or ("prefill", tile rows, (columns, 0, 0) of gate/up, (columns, 0, K split) of down)."""
+    import ctypes
+    P = pkg()
+    out = (ctypes.c_int32 * 8)()
+    P.lib().w4a16_internal_moe_route(3 if fmt == "prep" else P.FORMATS[fmt], T, K, I, E, topk, G, out)
+    return ("", "direct", "prefill")[out[0]], out[1], tuple(out[2:5]), tuple(out[5:8])
+
+
 def to_dev(a, device="cuda:0"):
     import torch
     a = np.ascontiguousarray(a)

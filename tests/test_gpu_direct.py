@@ -4,10 +4,12 @@ shares that its wave groups and workgroups do not divide evenly, every group siz
 type and instance (each case names its own, which a test without GPU holds it to). x holds whole numbers up to 2 in size and the scales are powers of two, so that
 every product and partial sum (below 2^24 units) is exact in fp32 in any order: the output must be
 the exact sum rounded once, bit for bit."""
+import math
+
 import numpy as np
 import pytest
 
-from helpers import pkg, route, to_dev
+from helpers import moe_route, pkg, route, to_dev
 from synth import Problem
 
 NAME = {0: "gptq", 1: "gptq_sym", 2: "awq"}
@@ -181,8 +183,10 @@ def test_plan_of_widths_other_kernels_do_not_tile():
 
 # ------------------------------------------------------------------ by expert
 
-FEW = [0, 1, 15, 16, 17, 32, 33, 48, 49, 64]                     # tiles of up to 64 rows
-MANY = [0, 1, 17, 49, 64, 65, 80, 81, 96, 97, 112, 113, 160, 225]  # up to 112 rows, one to three each
+# rows per expert, at the edges of 16-row blocks, of tiles of 64 and of 112 rows: one to four tiles each
+FEW = [0, 1, 15, 16, 17, 32, 33, 48, 49, 64]
+MANY = [0, 1, 17, 49, 64, 65, 80, 81, 96, 97, 112, 113, 160, 225]
+LONG = [65, 96, 97, 112, 160, 208]
 
 
 def expert_layer(counts, fmt, K, I, G, seed):
@@ -204,7 +208,8 @@ def expert_layer(counts, fmt, K, I, G, seed):
 @pytest.mark.parametrize("fmt,K,I,G", [(0, 512, 256, 64), (1, 256, 384, 64), (2, 256, 640, 128), (0, 256, 8192, 128),
                                        (2, 256, 8192, 64)])
 def test_direct_by_expert(torch_cuda, counts, fmt, K, I, G):
-    """Experts whose rows end at the edges of the tiles. With K in one chain the layer is the
+    """Experts whose rows end at the edges of the tiles, which are 64 rows high for these narrow layers
+    (test_direct_by_expert_tall: 112). With K in one chain the layer is the
     composition of the public pieces bit for bit; a long down projection (I = 8192) adds the sums of
     its wave groups in another order: within the fp32 rounding of the sums, two roundings of the
     16-bit results (h, y) and the weights' share: 2e-3 of the largest."""
@@ -212,6 +217,8 @@ def test_direct_by_expert(torch_cuda, counts, fmt, K, I, G):
     P = pkg()
     x, logits, w13, w2 = expert_layer(counts, fmt, K, I, G, 7 + fmt)
     args = dict(topk=1, fmt=NAME[fmt], group_size=G)
+    tiles = moe_route(NAME[fmt], sum(counts), K, I, len(counts), 1, G)
+    assert tiles == ("direct", 64, (7, 4, 1), (7, 4, 1) if I < 8192 else (4, 2, 4))
     y = P.fused_moe(x, logits, w13, w2, **args)
     again = P.fused_moe(x, logits, w13, w2, **args)
     want = _layer_by_pieces(P, x, logits, w13, w2, 1, NAME[fmt], G, 64)
@@ -221,6 +228,100 @@ def test_direct_by_expert(torch_cuda, counts, fmt, K, I, G):
     prep = [y] if fmt == 1 else [y, P.fused_moe_prepared(
         x, logits, *(P.prepare_layout_experts(*w, fmt=NAME[fmt], group_size=G) for w in (w13, w2)), topk=1)]
     for got in prep:
+        err = (got.float() - want.float()).abs().max() / want.float().abs().max()
+        assert err.item() <= 2e-3
+
+
+def random_layer(torch, counts, fmt, K, I, G, seed):
+    """As expert_layer, the weights' words and scales drawn on the device."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    E = len(counts)
+    ids = torch.repeat_interleave(torch.arange(E, device="cuda"), torch.tensor(counts, device="cuda"))
+    ids = ids[torch.randperm(len(ids), generator=g, device="cuda")]
+    x = torch.randn((len(ids), K), generator=g, device="cuda").half()
+    logits = torch.where(torch.arange(E, device="cuda") == ids[:, None], 4.0, 0.0)
+
+    def stack(rows, cols):
+        def words(*shape):
+            return torch.randint(-2 ** 31, 2 ** 31, shape, generator=g, device="cuda", dtype=torch.int64).int()
+        q = words(E, rows, cols // 8) if fmt == 2 else words(E, rows // 8, cols)
+        sc = torch.rand((E, rows // G, cols), generator=g, device="cuda") * 0.01 + 0.002
+        return q, sc.half(), None if fmt == 1 else words(E, rows // G, cols // 8)
+    return x, logits.float(), stack(K, 2 * I), stack(I, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,counts,K,I,G", [
+    (0, MANY, 2048, 1536, 128), (1, MANY, 2048, 1536, 64), (2, MANY, 2048, 1536, 128),
+    (0, LONG, 2048, 8192, 64), (2, LONG, 2048, 8192, 128)], ids=["gptq", "sym", "awq", "gptq-long", "awq-long"])
+def test_direct_by_expert_tall(torch_cuda, fmt, counts, K, I, G):
+    """Tiles of up to 112 rows, every height from one to seven 16-row blocks, the long down projection
+    over two wave groups. Equal to the pieces, or within the bounds of test_direct_by_expert."""
+    from test_gpu_moe import _layer_by_pieces
+    P = pkg()
+    down = (7, 4, 1) if I < 8192 else (7, 4, 2)
+    for f in (NAME[fmt], "prep"):
+        assert moe_route(f, sum(counts), K, I, len(counts), 1, G) == ("direct", 112, (7, 4, 1), down)
+    x, logits, w13, w2 = random_layer(torch_cuda, counts, fmt, K, I, G, 70 + fmt)
+    args = dict(topk=1, fmt=NAME[fmt], group_size=G)
+    y = P.fused_moe(x, logits, w13, w2, **args)
+    again = P.fused_moe(x, logits, w13, w2, **args)
+    want = _layer_by_pieces(P, x, logits, w13, w2, 1, NAME[fmt], G, 64)
+    assert torch_cuda.equal(y, again)
+    if I < 8192:
+        assert torch_cuda.equal(y, want)
+    prep = [] if fmt == 1 else [P.fused_moe_prepared(
+        x, logits, *(P.prepare_layout_experts(*w, fmt=NAME[fmt], group_size=G) for w in (w13, w2)), topk=1)]
+    for got in [y] + prep:
+        err = (got.float() - want.float()).abs().max() / want.float().abs().max()
+        assert err.item() <= 2e-3
+
+
+def test_expert_tiles_are_direct_or_of_256_rows():
+    """Over layers of every size: tiles of 64 or 112 rows on the direct kernel, of 256 on the prefill
+    kernel, there where they are over 0.83 full or an expert has over 1024 rows."""
+    seen = set()
+    for E in (1, 4, 8, 60, 256):
+        for T in (1, 5, 60, 400, 880, 1900, 3600, 8000):
+            for topk in (1, 2):
+                for K, I in ((256, 256), (1024, 896), (4096, 2048), (4096, 14336)):
+                    kind, rows, _, _ = moe_route("gptq", T, K, I, E, min(topk, E), 128)
+                    mean = T * min(topk, E) / E
+                    full = math.ceil((mean + math.sqrt(mean)) / 256)
+                    assert kind == ("prefill" if mean > 1024 or mean > 0.83 * 256 * full else "direct")
+                    seen.add((kind, rows))
+    assert seen == {("direct", 64), ("direct", 112), ("prefill", 256)}
+
+
+# 256-row tiles of the prefill kernel: rows of experts on average, experts, K, I; columns of gate/up, of
+# down, K split of down
+FULL = [(216, 4, 256, 512, 128, 128, 1), (216, 16, 256, 1792, 224, 128, 1), (216, 10, 256, 2048, 256, 128, 1),
+        (240, 4, 256, 8192, 256, 256, 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("mean,E,K,I,bn13,bn2,ks2", FULL)
+def test_expert_tiles_of_256_rows(torch_cuda, fmt, mean, E, K, I, bn13, bn2, ks2):
+    """Experts of about 216 or 240 rows, one of 256 and one just above: the prefill kernel's tiles.
+    Equal to the pieces where K is whole, else (and prepared) within the bounds above."""
+    from test_gpu_moe import _layer_by_pieces
+    P = pkg()
+    counts = [mean] * (E - 4) + [257, 256, 2 * mean - 257 + 16, 2 * mean - 256 - 16]
+    assert sum(counts) == mean * E
+    for f in (NAME[fmt], "prep"):
+        assert moe_route(f, mean * E, K, I, E, 1, 128) == ("prefill", 256, (bn13, 0, 0), (bn2, 0, ks2))
+    x, logits, w13, w2 = random_layer(torch_cuda, counts, fmt, K, I, 128, 90 + fmt)
+    args = dict(topk=1, fmt=NAME[fmt], group_size=128)
+    y = P.fused_moe(x, logits, w13, w2, **args)
+    again = P.fused_moe(x, logits, w13, w2, **args)
+    want = _layer_by_pieces(P, x, logits, w13, w2, 1, NAME[fmt], 128, 64)
+    assert torch_cuda.equal(y, again)
+    if ks2 == 1:
+        assert torch_cuda.equal(y, want)
+    prep = [] if fmt == 1 else [P.fused_moe_prepared(
+        x, logits, *(P.prepare_layout_experts(*w, fmt=NAME[fmt], group_size=128) for w in (w13, w2)), topk=1)]
+    for got in [y] + prep:
         err = (got.float() - want.float()).abs().max() / want.float().abs().max()
         assert err.item() <= 2e-3
 

@@ -203,19 +203,19 @@ def _layer_by_pieces(P, x, logits, w13, w2, topk, fmt, G, block_m):
     return P.moe_sum(yp, w, T, topk, K)
 
 
-# The fused layer computes its grouped GEMMs over expert tiles (an expert's rows in one tile
-# of 64/128/192/256 rows, 256/224/128 columns, chosen from the mean rows per expert and the CU
-# count). Every pair row goes through the same arithmetic as in the block_m-block GEMM, so
-# the layer must equal the composition of the public pieces bit for bit. Cases, with the
-# tiles they take on a 256-CU MI355X: (T, E, topk, K, I, skew, fmt, block_m)
+# The fused layer computes its grouped GEMMs over expert tiles: an expert's rows in tiles of up to
+# 64 or 112 rows on the direct kernel, as in all these cases, or of 256 on the prefill kernel
+# (test_gpu_direct.py holds layers to each of them). Every pair row goes through the same
+# arithmetic as in the block_m-block GEMM, so the layer must equal the composition of the public
+# pieces bit for bit. Cases: (T, E, topk, K, I, skew, fmt, block_m)
 TILE_CASES = [
-    (512, 8, 2, 256, 1792, None, GPTQ, 64),     # 192 x 224 (gate/up), 192 x 128 (down)
-    (512, 8, 2, 256, 4096, None, AWQ, 128),     # 192 x 256, 192 x 128
-    (512, 8, 2, 256, 256, 3, GPTQ, 64),         # expert 3 takes ~512 rows: 3 tiles of it
-    (300, 8, 2, 512, 256, 0, AWQ, 64),          # 128-row tiles, expert 0 in 3 of them
-    (1024, 4, 2, 256, 512, None, SYM, 128),     # 256-row tiles, two per expert
-    (48, 4, 2, 256, 256, None, AWQ, 64),        # 64-row tiles
-    (40, 64, 2, 256, 256, None, GPTQ, 64),      # 64-row tiles, most experts without tokens
+    (512, 8, 2, 256, 1792, None, GPTQ, 64),     # experts of about 128 rows
+    (512, 8, 2, 256, 4096, None, AWQ, 128),
+    (512, 8, 2, 256, 256, 3, GPTQ, 64),         # expert 3 takes ~512 rows
+    (300, 8, 2, 512, 256, 0, AWQ, 64),          # expert 0 takes ~300
+    (1024, 4, 2, 256, 512, None, SYM, 128),     # 512 rows each
+    (48, 4, 2, 256, 256, None, AWQ, 64),
+    (40, 64, 2, 256, 256, None, GPTQ, 64),      # most experts without tokens
 ]
 
 
@@ -249,8 +249,8 @@ def test_fused_layer_expert_tiles_equal_block_composition(torch_cuda, orc, case)
 
 @pytest.mark.parametrize("fmt", [GPTQ, AWQ])
 def test_fused_layer_down_projection_split_k(torch_cuda, fmt):
-    """A long down projection (I = 8192) splits its K over two workgroups per tile (fp32
-    partials summed in split order): the layer stays within the GEMM tolerance of the
+    """A long down projection (I = 8192) splits its K, here over the wave groups of a workgroup
+    (over two workgroups on the prefill kernel's tiles: test_gpu_direct.py): the layer stays within the GEMM tolerance of the
     block_m composition, and repeated calls are bit-identical."""
     T, E, topk, K, I, G = 512, 4, 2, 256, 8192, 128
     P = pkg()
@@ -348,7 +348,7 @@ def test_fused_moe_prepared_tile_cases(torch_cuda, orc, case):
 
 @pytest.mark.parametrize("fmt", [GPTQ, AWQ])
 def test_fused_moe_prepared_down_projection_split_k(torch_cuda, orc, fmt):
-    """I = 8192: the prepared down projection splits its K over two workgroups per tile."""
+    """I = 8192: the prepared down projection splits its K over wave groups."""
     T, E, topk, K, I, G = 512, 4, 2, 256, 8192, 128
     P = pkg()
     g = np.random.default_rng(190 + fmt)

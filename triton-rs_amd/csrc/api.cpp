@@ -1241,17 +1241,15 @@ MoeLayout moe_layout(int32_t T, int32_t E, int32_t topk, int32_t I, int32_t K, i
     return L;
 }
 
-// Expert-tile shape of the fused layer's grouped GEMMs. Tile height: the smallest of 64,
-// 128, 192, 256 rows holding 1.25x the mean rows per expert, so that one tile usually covers
-// all of an expert's tokens and its weights are dequantised once per column tile. Tile
-// width: the fewest rounds of workgroups over the CUs times the width (ties to the wider
-// tile), for the tile count a balanced routing gives; 64-row tiles come 256 wide only.
+// Expert-tile shape of the fused layer's grouped GEMMs on the prefill kernel: 256 rows, for experts that
+// fill them (moe_direct takes the others). Tile width: the fewest rounds of workgroups over the CUs times
+// the width (ties to the wider tile), for the tile count a balanced routing gives. Up to 51 rows per
+// expert the layer is taken in widths of whole 256-column tiles only.
 struct MoeTiles {
     int bm, bn13, bn2, ks2;
     DirectShape d13, d2;   // ok: this GEMM on the direct kernel
 };
-int moe_tile_bn(int N, int bm, int est_tiles, int cus) {
-    if (bm == 64) return 256;
+int moe_tile_bn(int N, int est_tiles, int cus) {
     int best = 0;
     long long best_cost = 0;
     for (int bn : {256, 224, 128}) {
@@ -1263,18 +1261,17 @@ int moe_tile_bn(int N, int bm, int est_tiles, int cus) {
     return best;
 }
 MoeTiles moe_tiles(int P, int E, int K, int I, int cus) {
-    const double want = 1.25 * P / E;
     MoeTiles t{};
-    t.bm = want <= 64 ? 64 : want <= 128 ? 128 : want <= 192 ? 192 : 256;
-    const int per_expert = (int)((P / E + t.bm - 1) / t.bm);
+    t.bm = 256;
+    const int per_expert = (P / E + t.bm - 1) / t.bm;
     const int est = E * (per_expert > 0 ? per_expert : 1);
-    t.bn13 = moe_tile_bn(2 * I, t.bm, est, cus);
-    t.bn2 = moe_tile_bn(K, t.bm, est, cus);
+    const bool few = 1.25 * P / E <= 64;
+    t.bn13 = few ? 256 : moe_tile_bn(2 * I, est, cus);
+    t.bn2 = few ? 256 : moe_tile_bn(K, est, cus);
     // down projection with 128-wide tiles and a long K: 256-wide tiles with K split in two
-    // (as the dense prefill does; config 4: 16 x 8 x 2 = 256 workgroups)
+    // (as the dense prefill does)
     t.ks2 = 1;
-    if (t.bn2 == 128 && t.bm > 64 && moe_down_may_split(K, I) &&
-        (long long)est * (K / 256) * 2 <= cus) {
+    if (t.bn2 == 128 && moe_down_may_split(K, I) && (long long)est * (K / 256) * 2 <= cus) {
         t.bn2 = 256;
         t.ks2 = 2;
     }
@@ -1308,6 +1305,19 @@ void moe_direct(MoeTiles& t, int fmt, int P, int T, int E, int K, int I, int G, 
     t = d;
 }
 }  // namespace
+
+// What the expert GEMMs of a fused layer run (as w4a16_internal_route), where its shape has expert tiles.
+// out: {1, tile rows, gate/up r, nwn, kw, down r, nwn, kw} the direct kernel; {2, tile rows, gate/up
+// columns, 0, 0, down columns, 0, K split of the down projection} the prefill kernel.
+W4A16_API void w4a16_internal_moe_route(int fmt, int32_t T, int32_t K, int32_t I, int32_t E, int32_t topk, int32_t G,
+                                        int32_t* out) {
+    const int cus = device_cus(), P = T * topk;
+    MoeTiles t = moe_tiles(P, E, K, I, cus);
+    moe_direct(t, fmt, P, T, E, K, I, G, cus);
+    const int32_t direct[8] = {1, t.bm, t.d13.r, t.d13.nwn, t.d13.kw, t.d2.r, t.d2.nwn, t.d2.kw},
+                  prefill[8] = {2, t.bm, t.bn13, 0, 0, t.bn2, 0, t.ks2};
+    for (int i = 0; i < 8; ++i) out[i] = t.d13.ok ? direct[i] : prefill[i];
+}
 
 W4A16_API size_t w4a16_fused_moe_workspace_size(int32_t T, int32_t E, int32_t topk, int32_t I,
                                                 int32_t K, int32_t block_m) {

@@ -902,14 +902,9 @@ static void launch_dma_t(const PrefillParams& p, dim3 grid, size_t lds, hipStrea
 template <int FMT, bool MOE, typename E = half_t>
 static void launch_dma_fmt(const PrefillParams& p, int bm, int bn, dim3 grid, size_t lds,
                            hipStream_t st) {
-    if constexpr (MOE) {
+    if constexpr (MOE) {   // 64 and 128 rows: blocks of the block_m grouped GEMM; 256: expert tiles
         if (bm == 64) launch_dma_t<FMT, 64, 256, true>(p, grid, lds, st);
-        else if (bm == 128 && bn == 224) launch_dma_t<FMT, 128, 224, true>(p, grid, lds, st);
-        else if (bm == 128 && bn == 128) launch_dma_t<FMT, 128, 128, true>(p, grid, lds, st);
         else if (bm == 128) launch_dma_t<FMT, 128, 256, true>(p, grid, lds, st);
-        else if (bm == 192 && bn == 224) launch_dma_t<FMT, 192, 224, true>(p, grid, lds, st);
-        else if (bm == 192 && bn == 128) launch_dma_t<FMT, 192, 128, true>(p, grid, lds, st);
-        else if (bm == 192) launch_dma_t<FMT, 192, 256, true>(p, grid, lds, st);
         else if (bn == 224) launch_dma_t<FMT, 256, 224, true>(p, grid, lds, st);
         else if (bn == 128) launch_dma_t<FMT, 256, 128, true>(p, grid, lds, st);
         else launch_dma_t<FMT, 256, 256, true>(p, grid, lds, st);
@@ -995,9 +990,7 @@ bool moe_tiles_supported(int N, int K, int G, long long a_rows, int bn) {
 
 hipError_t launch_moe_gemm_tiles(int fmt, const PrefillParams& p, int tile_bm, int bn,
                                  int max_tiles, hipStream_t st) {
-    const bool shape_ok = (tile_bm == 64 && bn == 256) || tile_bm == 128 || tile_bm == 192 ||
-                          tile_bm == 256;
-    if (!p.tiles || !p.num_tiles || !shape_ok ||
+    if (!p.tiles || !p.num_tiles || tile_bm != 256 ||
         !moe_tiles_supported(p.N, p.K, p.G, (p.num_pairs + p.a_div - 1) / p.a_div, bn))
         return hipErrorInvalidValue;
     if (p.ksplit > 1 && (!p.ws || !p.counters || (p.K / BK) % p.ksplit ||

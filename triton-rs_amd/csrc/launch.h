@@ -130,8 +130,8 @@ hipError_t launch_prefill(int fmt, const PrefillParams& p, const PrefillShape& s
 bool moe_gemm_supported(int N, int K, int G, int block_m);
 hipError_t launch_moe_gemm(int fmt, const PrefillParams& p, int block_m, int max_blocks,
                            hipStream_t st);
-// Expert-tile grouped GEMM: tile rows tile_bm (128, 192 or 256 with tile columns bn = 256,
-// 224 or 128 dividing N; 64 with bn = 256); grid rows max_tiles, the bound of moe_max_tiles.
+// Expert-tile grouped GEMM: tiles of tile_bm = 256 rows and bn = 256, 224 or 128 columns dividing N;
+// grid rows max_tiles, the bound of moe_max_tiles.
 bool moe_tiles_supported(int N, int K, int G, long long a_rows, int bn);
 hipError_t launch_moe_gemm_tiles(int fmt, const PrefillParams& p, int tile_bm, int bn,
                                  int max_tiles, hipStream_t st);
