@@ -277,6 +277,12 @@ PMC_WORKLOADS = {
     "prepstored_c2_m16": ("gptq", 16, 4096, 6144, 128, True),
     "prepstored_c2_m32": ("gptq", 32, 4096, 6144, 128, True),
     "prepstored_c2_m64": ("gptq", 64, 4096, 6144, 128, True),
+    # the kernel that dequantises in registers: a decode batch, a chunk (also in bfloat16), and
+    # config 4's layer with 16 tokens
+    "m48_k4096_n28672": ("awq", 48, 4096, 28672, 128, False),
+    "m200_k4096_n28672": ("gptq", 200, 4096, 28672, 128, False),
+    "bf16_m200_k4096_n28672": ("gptq", 200, 4096, 28672, 128, False),
+    "moe_t16": None,
 }
 
 
@@ -286,10 +292,10 @@ def c2_g_idx(torch, dev, K=4096, G=128):
     return (torch.arange(K) // G)[perm].to(torch.int32).to(dev)
 
 
-def moe_layer(torch, dev, gen):
-    """Config 4's layer: T=512 tokens, 8 experts, top-2, K=4096, I=14336, GPTQ G=128, random
+def moe_layer(torch, dev, gen, T=512):
+    """Config 4's layer: T=512 tokens (or as given), 8 experts, top-2, K=4096, I=14336, GPTQ G=128, random
     packed words, scales in [0.002, 0.02], fp32 router logits ~ N(0, 1)."""
-    T, E, topk, K, I, G = 512, 8, 2, 4096, 14336, 128
+    E, topk, K, I, G = 8, 2, 4096, 14336, 128
 
     def words(*shape):
         return torch.randint(-2 ** 31, 2 ** 31 - 1, shape, dtype=torch.int32, device=dev, generator=gen)
@@ -313,10 +319,10 @@ def pmc_child(args) -> int:
     import __graft_entry__
     pkg = __graft_entry__.load_package()
     dev = torch.device("cuda:0")
-    if args.pmc_workload == "c4_moe":
+    if PMC_WORKLOADS[args.pmc_workload] is None:
         gen = torch.Generator(device=dev)
         gen.manual_seed(0x5EED0004)
-        L = moe_layer(torch, dev, gen)
+        L = moe_layer(torch, dev, gen, T=16 if args.pmc_workload == "moe_t16" else 512)
         out = torch.empty((L["T"], L["K"]), dtype=torch.float16, device=dev)
         for _ in range(PMC_WARM + PMC_MEASURED):
             pkg.fused_moe(L["x"], L["logits"], L["w13"], L["w2"], topk=L["topk"], out=out)
@@ -326,8 +332,10 @@ def pmc_child(args) -> int:
         n_sets = args.sets if M <= 64 else 2
         sets = make_weight_sets(torch, fmt, K, N, G, n_sets, dev, seed=0x5EED0001)
         g_idx = c2_g_idx(torch, dev, K, G) if act_order else None
-        x = torch.randn((M, K), device=dev).half()
-        out = torch.empty((M, N), dtype=torch.float16, device=dev)
+        dt = torch.bfloat16 if args.pmc_workload.startswith("bf16_") else torch.float16
+        x = torch.randn((M, K), device=dev).to(dt)
+        sets = [(qw, sc.to(dt), qz) for qw, sc, qz in sets]
+        out = torch.empty((M, N), dtype=dt, device=dev)
         if args.pmc_workload.startswith("prepstored_"):
             prep = [pkg.prepare_layout(qw, sc, qz, fmt=fmt, group_size=G, zero_offset=1)
                     for qw, sc, qz in sets]

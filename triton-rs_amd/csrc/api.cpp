@@ -227,8 +227,10 @@ static bool act_order_chunks_ok(int fmt, int M, int N, int K, int G) {
 // split of K (4096 -> 28672 M = 16 / 32 / 48 24.5 / 30.5 / 46.7 -> 18.6 / 22.5 / 24.8 us; below,
 // 4096 -> 6144 M = 16 / 48 8.8 / 13.9 us against 10.3 / 15.0; in bf16 from 17 rows, 16 rows 20.7 us
 // against 23.6 on 4096 -> 20480). In fp16 also 4 rows from K = 4096, where the VALU GEMV's dot products
-// cost more (4 rows, 4096 -> 20480 / 28672, 8192 -> 28672 20.5 / 27.7 / 49.0 -> 19.5 / 21.7 / 39.7 us;
-// 2 rows 16.4 us against 21.5; 5 and 8 rows, split-K kernel, 4096 -> 20480 16.7 / 16.9 against 19.5).
+// cost more. VALU GEMV, direct: 4 rows 4096 -> 20480 / 24576 / 28672 / 40960 20.1 / 23.1 / 26.0 / 34.8, 19.3 /
+// 19.6 / 19.7 / 28.2 us, 8192 -> 20480 / 28672 34.5 / 46.5, 29.1 / 35.2; 3 rows 14.9 / 18.9 / 21.1 / 27.8, 19.4 /
+// 19.7 / 19.9 / 28.2 and 25.2 / 36.4, 29.5 / 35.2, so a rule for 3 would win 6 % and lose 30; from 5 rows the
+// split-K small-batch kernel: 8 rows 16.7 / 17.1 / 23.0 / 23.7 and 26.4 / 34.3.
 // Widths no tile of the others divides came to the generic kernel before; narrow ones (N < 512) stay there.
 static DirectShape direct_choice(int fmt, int M, int N, int K, int G, int cus, bool bf16,
                                  size_t max_partial_bytes = SIZE_MAX, size_t max_tiles = SPLITK_MAX_TILES) {
@@ -1282,7 +1284,8 @@ MoeTiles moe_tiles(int P, int E, int K, int I, int cus) {
 // fill the chip. It dequantises a weight once per such tile, the prefill kernel once per 256 rows, and
 // computes 16-row blocks, where the prefill kernel computes its whole tile: so it stays out where
 // tiles of 256 rows would be over 0.83 full.
-// Measured per layer (8 experts, top 2, K = 4096, I = 14336, GPTQ; prefill tiles, direct): 4 / 16 /
+// Measured per layer (8 experts, top 2, K = 4096, I = 14336, GPTQ; the best prefill tiles of 64 to 256
+// rows, direct): 4 / 16 /
 // 64 tokens 358 / 416 / 446, 149 / 192 / 200 us; 256 / 512 / 640 / 832 / 1024 tokens 477 / 556 /
 // 622 / 711 / 1037, 338 / 473 / 532 / 647 / 858 us; 864 / 960 / 1792 / 1920 (0.84 to 0.94 full)
 // 714 / 745 / 1312 / 1351, 762 / 822 / 1348 / 1484 us; 1536 / 3072 / 5000 / 8000 1181 / 2522 / 3751 /

@@ -20,10 +20,12 @@
 // v_perm and two shifts put a byte into both halves of a register, v_and_or makes (1024 + q,
 // 1024 + 16 q'), v_pk_fma gives (q - z, q' - z) exactly, v_pk_mul rounds (q - z) s once), 8 R
 // MFMAs and 50 others; measured 0.42 to 0.88 us (R = 1 to 7) against 0.33 to 0.62 us of issue.
-// Measured (K = 4096, GPTQ, 20 weight sets in turn; before: the prefill kernel, from 48 rows down
-// the small-batch kernels): N = 6144: M = 128 / 200 / 512 / 1024 32.3 / 38.7 / 51.0 / 76.3 ->
-// 19.6 / 24.4 / 38.0 / 62.1 us; N = 28672: M = 16 / 48 / 200 24.6 / 46.7 / 74.5 -> 18.6 / 24.8 /
-// 60.8 us; AWQ M = 48: N = 4096 / 6144 / 28672 25.0 / 25.5 / 42.4 -> 12.5 / 14.0 / 27.8 us.
+// Counters (K = 4096, N = 28672, one wave per SIMD): of a wave's time 59 % issuing and 20 % waiting
+// for its turn at 48 rows of AWQ, 64 and 18 % at 200 of GPTQ, 73 and 15 % in bf16 (254 VALU a stage).
+// Measured (K = 4096, GPTQ, weight sets in turn; before: the prefill kernel, from 48 rows down the
+// small-batch kernels): N = 6144: M = 128 / 200 / 512 / 1024 / 2048 30.8 / 37.0 / 47.7 / 72.5 / 107.3 ->
+// 19.0 / 22.3 / 34.4 / 58.1 / 101.4 us; N = 28672: M = 16 / 48 / 200 24.6 / 46.7 / 69.4 -> 18.6 / 24.8 /
+// 55.9 us; AWQ M = 48: N = 4096 / 6144 / 28672 25.0 / 25.5 / 42.4 -> 12.5 / 14.0 / 27.8 us.
 #pragma once
 #include <type_traits>
 
@@ -546,8 +548,8 @@ __global__ void __launch_bounds__(64 * NWN * KW, 2) direct_kernel(PrefillParams 
     direct_tile<FMT, E, R, NWN, KW, false>(p, lds, ct, rt, bz, rt * 16 * R, min(16 * R, p.M - rt * 16 * R));
 }
 
-// 8 experts of 4096 -> 28672 and 14336 -> 4096, top 2: 16 tokens 228 + 182 -> 120 + 61 us (traced;
-// the weights alone take 92 + 46 at the rate of a large copy), 512 tokens 422 + 203 -> 300 + 197 us.
+// 8 experts of 4096 -> 28672 and 14336 -> 4096, top 2: 16 tokens 228 + 182 -> 124 + 63 us (traced;
+// the weights alone take 92 + 46 at the rate of a large copy), 512 tokens 422 + 203 -> 318 + 176 us.
 // Grouped by expert: row tile rt is entry rt of the tile list ({first sorted row, rows, expert, 0});
 // the tile's rows, known on the device only, pick the code for their number of 16-row blocks, so
 // that a tile costs what its rows need. The K groups' LDS must hold 16 RMAX rows.
