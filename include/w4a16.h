@@ -102,12 +102,13 @@ W4A16_API int w4a16_init(int32_t device);
  * retires the old one without freeing it (HIP graphs captured earlier keep using it), so a
  * captured call stays valid for the life of the process. Growing the workspace is not
  * possible under stream capture: make one call of the largest size before capturing, or
- * the call fails with W4A16_ERR_UNSUPPORTED. Concurrent calls on different streams are
+ * the call fails with W4A16_ERR_UNSUPPORTED (or, on the kernel that dequantises in registers,
+ * runs with the splits of K that the workspace holds, down to none). Concurrent calls on different streams are
  * safe. With g_idx from 65 to 128 rows (GPTQ formats, K <= 4096) the small-batch kernel runs
  * in two row chunks; beyond that (K <= 32768, K / group_size <= 1024) each
  * call also computes the group order of the rows on the device, repacks the rows and gathers
- * x into per-(device, stream) buffers (grown like the workspace) and runs the prefill
- * kernel on them; when g_idx's groups do not each hold exactly group_size rows (or an entry
+ * x into per-(device, stream) buffers (grown like the workspace) and runs the plain-order
+ * kernel for its rows on them; when g_idx's groups do not each hold exactly group_size rows (or an entry
  * is out of range) the generic kernel runs instead, decided on the device. */
 W4A16_API int w4a16_gemm(void* stream, int fmt, const void* x, const void* qweight,
                          const void* scales, const void* qzeros, const int32_t* g_idx,
